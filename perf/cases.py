@@ -304,6 +304,9 @@ def _captured(step):
 
 
 def prepare(case: dict, seed: int) -> dict:
+    from moelab_hip import _lib
+
+    _lib.check_device(DEV)  # a program's set-up call (probes the device once)
     kind = case["kind"]
     if kind == "dense":
         return _prepare_dense(case, seed)
