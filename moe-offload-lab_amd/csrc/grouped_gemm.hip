@@ -16,18 +16,30 @@
 // n - 8 (exact) and s * (n - 8) (one fp16 rounding, relative error <= 2^-11; the reference's own
 // prefill path rounds the dequantised weights to the model dtype, 2^-8 for bf16).
 //
-// Operand A is fp16 in LDS: fp16 activations as they are, bf16 activations scaled per token by a
-// power of two 2^-e (the row's largest |x| in [2^14, 2^15), exact for bf16 values), h (fp32,
-// written by the up kernel with a per-pair maximum gathered by atomics) scaled per pair the
-// same way; the outputs are scaled back by 2^e.
+// Operand A is fp16 in operand order (see AStage): fp16 activations as they are, bf16 activations
+// scaled per token by a power of two 2^-e (the row's largest |x| in [2^14, 2^15), exact for bf16
+// values); h (written fp16 by the up tiles) carries a power of two per (pair, 32 columns); the
+// outputs are scaled back.
 //
-// Each workgroup (4 waves) owns one expert and 256 weight rows (up: 128 gate + 128 up rows =
-// 128 h columns; down: 256 output rows); a wave owns 2 subtiles of 32 rows, for up to 64
-// tokens per pass (two 32-token M tiles). K advances in chunks (up: 4 groups, down: 2): a wave
-// keeps a ring of chunks of its weight rows in registers (16 KB in flight while it computes),
-// and the workgroup stages the activation chunk into LDS (double buffered, rows padded by 16
-// bytes, permuted into operand order) one chunk ahead. Workgroups of one expert land on one XCD
-// (its L2 then serves the expert's activation rows to all of them).
+// Each workgroup (4 waves) owns one work unit (an expert's pass of up to 64 or 128 of its pairs,
+// see gg_units) and 256 weight rows (up: 128 gate + 128 up rows = 128 h columns; down: 256 output
+// rows); a wave owns 2 subtiles of 32 rows. K advances in chunks of 64 bytes of a weight row: a
+// wave holds two chunks of its weight rows in registers, the activation chunks are copied from
+// memory straight into LDS. Workgroups of one unit land on one XCD (its L2 then serves the unit's
+// activation rows to all of them).
+//
+// What bounds it and what it measured (us per launch, up / down, before = 64-token passes in a chain
+// per expert, activations staged through registers, 2 workgroups per CU everywhere):
+//   fp8, 512 experts (d_model 2048, d_ff 512) + a shared expert, 333 tokens: 408 / 207 -> 234 / 127;
+//     the weights (1.61 GB) take 315 of these 361 at the 5.1 TB/s of a large copy. Three things:
+//     the shared expert's 333 tokens were one workgroup's chain of six passes at the end of the grid,
+//     a chunk's activations waited for the weights issued before them, 20 operations per 8 weights.
+//   int4, 64 experts (d_ff 1024), 2048 tokens: 270 / 165 -> 193 / 123; MFMA busy 40 %, the clock at
+//     2.06 of 2.4 GHz; the conversion's VALU work is 42 % of the SIMD's time (128 tokens per pass
+//     halve it per token; interleaving it with the MFMAs by hand changed nothing).
+//   int4, 128 experts (d_ff 768), 512 tokens: 87 / 52 -> 71 / 48 for 201 / 101 MB of weights; the same
+//     loop without MFMAs and conversion takes 59 / 34, without the activation copies too 55, a bare
+//     read of the weights 38.
 
 #include "decide.hpp"
 #include "lanevec.hpp"
@@ -53,6 +65,7 @@ template <int CKV> struct GgChunk {
     static constexpr int VPT = CK / 4;      // values staged per thread
     static constexpr int NV = VPT / 8;      // 16-byte loads per thread
 };
+template <int N> struct IntC { static constexpr int value = N; };
 template <int PREC> struct GgPrec;
 template <> struct GgPrec<MOEHIP_PREC_INT4> { static constexpr int CK = 128, BITS = 4; };
 template <> struct GgPrec<MOEHIP_PREC_INT8> { static constexpr int CK = 64, BITS = 8; };
@@ -107,19 +120,19 @@ __device__ __forceinline__ f16x8 wdeq8_i8(uint32_t lo, uint32_t hi, half2_t s2) 
     return __builtin_bit_cast(f16x8, make_uint4(r[0], r[1], r[2], r[3]));
 }
 
-// fp8 e4m3fn: pair i moved into the HIGH bytes of two halves (b << 8); (v & sign) | ((v >> 1) &
-// 0x3F80) is the fp16 of value * 2^-8 exactly (exponent bias 15 vs 7, subnormals included; the
-// format's only NaN code never occurs in a record), * fp16(block scale * 2^8) (one rounding).
+// fp8 e4m3fn: the bytes put into operand order by two v_perm_b32, each pair converted to the fp16
+// of value * 2^-8 exactly by v_cvt_scalef32_pk_f16_fp8 (scale 2^-8; subnormals included), * fp16(
+// block scale * 2^8) (one rounding). 10 operations per 8 weights; the shift-and-mask form took 20.
 __device__ __forceinline__ f16x8 wdeq8_fp8(uint32_t lo, uint32_t hi, half2_t s2) {
-    uint32_t r[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const uint32_t sel = 0x000C000Cu | ((uint32_t)(4 + i) << 24) | ((uint32_t)i << 8);
-        const uint32_t v = __builtin_amdgcn_perm(hi, lo, sel);
-        const uint32_t u = and_or(v >> 1, 0x3F803F80u, v & 0x80008000u);
-        r[i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, u) * s2);
-    }
-    return __builtin_bit_cast(f16x8, make_uint4(r[0], r[1], r[2], r[3]));
+    const int p0 = (int)__builtin_amdgcn_perm(hi, lo, 0x05010400u);  // c0 c4 c1 c5
+    const int p1 = (int)__builtin_amdgcn_perm(hi, lo, 0x07030602u);  // c2 c6 c3 c7
+    const half2_t h0 = (half2_t)__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(p0, 0.00390625f, false) * s2;
+    const half2_t h1 = (half2_t)__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(p0, 0.00390625f, true) * s2;
+    const half2_t h2 = (half2_t)__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(p1, 0.00390625f, false) * s2;
+    const half2_t h3 = (half2_t)__builtin_amdgcn_cvt_scalef32_pk_f16_fp8(p1, 0.00390625f, true) * s2;
+    const uint4 u = make_uint4(__builtin_bit_cast(uint32_t, h0), __builtin_bit_cast(uint32_t, h1),
+                               __builtin_bit_cast(uint32_t, h2), __builtin_bit_cast(uint32_t, h3));
+    return __builtin_bit_cast(f16x8, u);
 }
 
 // fp16 / bf16: halves c0..c7 in dwords d0..d3; pair i = (c_i, c_i+4) by one v_perm_b32; bf16 pairs
@@ -141,112 +154,82 @@ __device__ __forceinline__ f16x8 wdeq8_16(uint32_t d0, uint32_t d1, uint32_t d2,
     return __builtin_bit_cast(f16x8, make_uint4(r[0], r[1], r[2], r[3]));
 }
 
-// one chunk of weights in registers: per subtile this lane half's 32 bytes of its row and the
-// raw scale (int4 / int8: fp16 group scale bits; fp8: fp32 block scale bits; fp16 / bf16: none)
+// one chunk of weights in registers: per subtile this lane half's 32 bytes of its row
 struct WChunk {
     uint4 q[2][2];
-    uint32_t s[2];
+};
+// the raw scales of two chunks (c even, c + 1) per subtile, one load each: int4: a dword per chunk
+// (the groups of its two lane halves); int8: the two chunks' fp16 scales in s[t][0]; fp8: the
+// block's fp32 scale in s[t][0]; fp16 / bf16: none. (A 2-byte load per chunk and subtile instead
+// cost a fifth of the weight stream: 47 against 39 us for 201 MB read in this pattern.)
+struct WScale {
+    uint32_t s[2][2];
 };
 
-// qp[t]: the lane's row (subtile t) + 32 * half; sp[t]: its scale row (see gemm_rows)
-template <int PREC>
-__device__ __forceinline__ void load_chunk(WChunk &w, gu8 *const (&qp)[2], gu8 *const (&sp)[2], int c) {
+// chunk c at the uniform field base qb, qo[t]: the lane's row (subtile t) + 32 * half
+__device__ __forceinline__ void load_chunk(WChunk &w, gu8 *qb, const uint32_t (&qo)[2], int c) {
+    gu8 *q = qb + (size_t)c * 64;  // 64 bytes of a row per chunk for every precision
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-        gu8 *q = qp[t] + (size_t)c * 64;  // 64 bytes of a row per chunk for every precision
-        w.q[t][0] = gld16(q);
-        w.q[t][1] = gld16(q + 16);
-        if constexpr (PREC == MOEHIP_PREC_INT4)
-            w.s[t] = *(const __attribute__((address_space(1))) uint16_t *)(sp[t] + (size_t)c * 4);
-        else if constexpr (PREC == MOEHIP_PREC_INT8)
-            w.s[t] = *(const __attribute__((address_space(1))) uint16_t *)(sp[t] + (size_t)c * 2);
-        else if constexpr (PREC == MOEHIP_PREC_FP8)
-            w.s[t] = *(const __attribute__((address_space(1))) uint32_t *)(sp[t] + (size_t)(c >> 1) * 4);
-        else
-            w.s[t] = 0u;
+        w.q[t][0] = gld16(q + qo[t]);
+        w.q[t][1] = gld16(q + qo[t] + 16);
+    }
+}
+// scales of chunks c (even) and c + 1 <= cl; EVEN: the row has an even number of chunks (int4 rows
+// of an odd multiple of 128 have not: their last pair is one chunk, and no byte past it is read)
+template <int PREC, bool EVEN>
+__device__ __forceinline__ void load_scales(WScale &w, gu8 *sb, const uint32_t (&so)[2], int c, int cl) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        if constexpr (PREC == MOEHIP_PREC_INT4) {
+            if constexpr (EVEN) {
+                const u32x2_t v = *(const __attribute__((address_space(1))) u32x2_t *)(sb + (size_t)c * 4 + so[t]);
+                w.s[t][0] = v.x, w.s[t][1] = v.y;
+            } else {
+                w.s[t][0] = gld4(sb + (size_t)c * 4 + so[t]);
+                w.s[t][1] = gld4(sb + (size_t)min(c + 1, cl) * 4 + so[t]);
+            }
+        } else if constexpr (PREC == MOEHIP_PREC_INT8) {
+            w.s[t][0] = gld4(sb + (size_t)c * 2 + so[t]);
+        } else if constexpr (PREC == MOEHIP_PREC_FP8) {
+            w.s[t][0] = gld4(sb + (size_t)(c >> 1) * 4 + so[t]);
+        }
     }
 }
 
-// row pointers of one lane: q row `row` of a (rows, K) weight matrix at qb, offset by the lane
-// half's 32 bytes; scale row at sb (int4 / int8: fp16 (rows, K / 64); fp8: fp32 (rows / 128,
-// K / 128) blocks)
+// byte offsets of one lane in a (rows, K) weight matrix's fields: its row + the lane half's 32
+// bytes; its scale row (int4 / int8: fp16 (rows, K / 64); fp8: fp32 (rows / 128, K / 128) blocks)
 template <int PREC>
-__device__ __forceinline__ void gemm_rows(gu8 *qb, gu8 *sb, int row, int K, int h, gu8 *&q, gu8 *&sc) {
-    q = qb + (size_t)row * ((size_t)K * GgPrec<PREC>::BITS / 8) + 32 * h;
-    if constexpr (PREC == MOEHIP_PREC_INT4) sc = sb + (size_t)row * (K / GG_KG) * 2 + 2 * h;
-    else if constexpr (PREC == MOEHIP_PREC_INT8) sc = sb + (size_t)row * (K / GG_KG) * 2;
-    else if constexpr (PREC == MOEHIP_PREC_FP8) sc = sb + (size_t)(row >> 7) * (K >> 7) * 4;
-    else sc = sb;
+__device__ __forceinline__ void gemm_rows(int row, int K, int h, uint32_t &qo, uint32_t &so) {
+    qo = (uint32_t)row * (uint32_t)(K * GgPrec<PREC>::BITS / 8) + 32u * h;
+    if constexpr (PREC == MOEHIP_PREC_INT4 || PREC == MOEHIP_PREC_INT8) so = (uint32_t)row * (K / GG_KG) * 2;
+    else if constexpr (PREC == MOEHIP_PREC_FP8) so = (uint32_t)(row >> 7) * (K >> 7) * 4;
+    else so = 0u;
+}
+
+// the scale of chunk parity U as an fp16 pair
+template <int PREC, int U>
+__device__ __forceinline__ half2_t scale_of(const uint32_t (&s)[2], int h) {
+    if constexpr (PREC == MOEHIP_PREC_INT4) {
+        return __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(s[U], s[U], h ? 0x03020302u : 0x01000100u));
+    } else if constexpr (PREC == MOEHIP_PREC_INT8) {
+        return __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(s[0], s[0], U ? 0x03020302u : 0x01000100u));
+    } else if constexpr (PREC == MOEHIP_PREC_FP8) {
+        const uint32_t sw = f32_to_f16_rne(__uint_as_float(s[0]) * 256.0f);
+        return __builtin_bit_cast(half2_t, sw | (sw << 16));
+    } else {
+        return half2_t{};
+    }
 }
 
 // B operand of MFMA step m of a chunk for one subtile (the lane's 8 dwords, natural K order)
 template <int PREC, int M>
-__device__ __forceinline__ f16x8 b_operand(const uint4 (&q)[2], uint32_t sraw, DeqK dk) {
+__device__ __forceinline__ f16x8 b_operand(const uint4 (&q)[2], half2_t s2, DeqK dk) {
     const uint32_t dw[8] = {q[0].x, q[0].y, q[0].z, q[0].w, q[1].x, q[1].y, q[1].z, q[1].w};
-    if constexpr (PREC == MOEHIP_PREC_INT4) {
-        const uint32_t sw = sraw & 0xffffu;
-        return wdeq8(dw[M], __builtin_bit_cast(half2_t, sw | (sw << 16)), dk);
-    } else if constexpr (PREC == MOEHIP_PREC_INT8) {
-        const uint32_t sw = sraw & 0xffffu;
-        return wdeq8_i8(dw[2 * M], dw[2 * M + 1], __builtin_bit_cast(half2_t, sw | (sw << 16)));
-    } else if constexpr (PREC == MOEHIP_PREC_FP8) {
-        const uint32_t sw = f32_to_f16_rne(__uint_as_float(sraw) * 256.0f);
-        return wdeq8_fp8(dw[2 * M], dw[2 * M + 1], __builtin_bit_cast(half2_t, sw | (sw << 16)));
-    } else {
-        return wdeq8_16<PREC>(dw[4 * M], dw[4 * M + 1], dw[4 * M + 2], dw[4 * M + 3]);
-    }
-}
-
-// ---------------------------------------------------------------------------------------
-// activation chunks (fp16): thread tid stages token tid / 4 of the pass, values VPT * (tid % 4) ..
-// of the chunk, permuted per 8 values into operand order (c0 c4 c1 c5 c2 c6 c3 c7), into LDS row
-// `tok`. Threads past the pass's tokens load a valid row too (no branch around the loads, which
-// keeps the compiler's load counting exact): MFMA rows are independent and those rows are never
-// stored.
-// ---------------------------------------------------------------------------------------
-template <int CK>
-__device__ __forceinline__ void xs_load(const uint16_t *row, int c, uint4 (&v)[GgChunk<CK>::NV]) {
-    const uint4 *p = reinterpret_cast<const uint4 *>(row + (size_t)c * CK + (threadIdx.x & 3) * GgChunk<CK>::VPT);
-#pragma unroll
-    for (int m = 0; m < GgChunk<CK>::NV; ++m) v[m] = p[m];
-}
-
-template <int CK>
-__device__ __forceinline__ void xs_store(const uint4 (&v)[GgChunk<CK>::NV], uint16_t *s_a) {
-    const int tok = threadIdx.x >> 2, part = threadIdx.x & 3;
-    uint4 *dst = reinterpret_cast<uint4 *>(s_a + tok * GgChunk<CK>::LDA + part * GgChunk<CK>::VPT);
-#pragma unroll
-    for (int m = 0; m < GgChunk<CK>::NV; ++m) {
-        const uint4 u = v[m];
-        dst[m] = make_uint4(lo_lo(u.x, u.z), hi_hi(u.x, u.z), lo_lo(u.y, u.w), hi_hi(u.y, u.w));
-    }
-}
-
-// ---------------------------------------------------------------------------------------
-// one chunk of MFMAs for a wave: CK / 16 steps x NM M tiles x 2 subtiles. Step m of lane half h
-// covers K h * CK / 2 + 8 m .. + 7 of the chunk, in A (LDS) and B (registers) alike.
-// ---------------------------------------------------------------------------------------
-template <int PREC, int NM, int M = 0>
-__device__ __forceinline__ void mma_steps(const WChunk &w, const uint16_t *ap, DeqK dk, f32x16 (&d)[2][2]) {
-    constexpr int CK = GgPrec<PREC>::CK;
-    if constexpr (M < CK / 16) {
-        const f16x8 b0 = b_operand<PREC, M>(w.q[0], w.s[0], dk);
-        const f16x8 b1 = b_operand<PREC, M>(w.q[1], w.s[1], dk);
-#pragma unroll
-        for (int mt = 0; mt < NM; ++mt) {
-            const f16x8 a = *reinterpret_cast<const f16x8 *>(ap + mt * 32 * GgChunk<CK>::LDA + 8 * M);
-            d[mt][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b0, d[mt][0], 0, 0, 0);
-            d[mt][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b1, d[mt][1], 0, 0, 0);
-        }
-        mma_steps<PREC, NM, M + 1>(w, ap, dk, d);
-    }
-}
-
-template <int PREC, int NM>
-__device__ __forceinline__ void mma_chunk(const WChunk &w, const uint16_t *s_a, DeqK dk, f32x16 (&d)[2][2]) {
-    constexpr int CK = GgPrec<PREC>::CK;
-    const int lane = threadIdx.x & 63, i = lane & 31, h = lane >> 5;
-    mma_steps<PREC, NM>(w, s_a + i * GgChunk<CK>::LDA + h * (CK / 2), dk, d);
+    if constexpr (PREC == MOEHIP_PREC_INT4) return wdeq8(dw[M], s2, dk);
+    else if constexpr (PREC == MOEHIP_PREC_INT8) return wdeq8_i8(dw[2 * M], dw[2 * M + 1], s2);
+    else if constexpr (PREC == MOEHIP_PREC_FP8) return wdeq8_fp8(dw[2 * M], dw[2 * M + 1], s2);
+    else return wdeq8_16<PREC>(dw[4 * M], dw[4 * M + 1], dw[4 * M + 2], dw[4 * M + 3]);
 }
 
 // fp16 bits of 2^d for d <= 0 (subnormal below 2^-14, 0 below 2^-24)
@@ -254,81 +237,252 @@ __device__ __forceinline__ uint32_t pow2_h(int d) {
     return d >= -14 ? (uint32_t)(d + 15) << 10 : (d >= -24 ? 1u << (d + 24) : 0u);
 }
 
-// h chunks staged by the down tiles: h is fp16 scaled by 2^-eb per (pair, 32 columns) (the up
-// wave of those columns chose eb); a staging thread multiplies its part of a chunk (CK / 4
-// columns, within one block of 32) by 2^(eb - emax), emax the pair's largest eb (exact unless the
-// product is subnormal), so one power per pair remains
-template <int CK>
-__device__ __forceinline__ void xs_scale(uint4 (&v)[GgChunk<CK>::NV], int eb, int emax) {
-    const uint32_t fb = pow2_h(eb - emax);
-    const half2_t f2 = __builtin_bit_cast(half2_t, fb | (fb << 16));
-#pragma unroll
-    for (int m = 0; m < GgChunk<CK>::NV; ++m) {
-        v[m].x = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, v[m].x) * f2);
-        v[m].y = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, v[m].y) * f2);
-        v[m].z = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, v[m].z) * f2);
-        v[m].w = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, v[m].w) * f2);
-    }
+// ---------------------------------------------------------------------------------------
+// activation chunks (fp16, already in operand order c0 c4 c1 c5 c2 c6 c3 c7 per 8 values): copied
+// straight from memory into LDS by buffer_load ... lds, 1 KB per instruction (no registers, no
+// VALU). (The global_load_lds form counts as a flat access: with one in flight the compiler waits
+// for every outstanding load before it uses the result of any.)
+// A chunk's LDS image is rows of CK values without padding; the 16-byte block b of row r sits at
+// block b ^ swz(r), so that the 32 rows an A operand reads at one K position fall on distinct
+// banks. The copy writes LDS in lane order, so the swizzle is in the address each lane reads.
+// ---------------------------------------------------------------------------------------
+template <int CK> struct AStage {
+    static constexpr int BPR = CK / 8;    // 16-byte blocks per row
+    static constexpr int RPI = 64 / BPR;  // rows per copy instruction
+    static __device__ __forceinline__ int swz(int r) { return (r / (16 / BPR)) & (BPR - 1); }
+    // copy instructions per wave for NM tiles of 32 tokens (4 waves share them; when there are
+    // fewer than 4, two waves copy the same rows: the same bytes to the same place)
+    static constexpr int total(int nm) { return nm * 32 / RPI; }
+    static constexpr int per_wave(int nm) { return (total(nm) + 3) / 4; }
+};
+
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+// a buffer of `bytes` bytes at the uniform address p (reads past it return 0)
+__device__ __forceinline__ rsrc_t buffer_of(const void *p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc((void *)(uintptr_t)uni64((int64_t)(uintptr_t)p), 0, uni((int)bytes), 0x00027000);
+}
+// 16 bytes per lane from byte off (per lane) + soff (uniform) of the buffer to dst + 16 * lane
+__device__ __forceinline__ void lds_copy16(rsrc_t buf, uint32_t off, uint32_t soff, uint16_t *dst) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, (__attribute__((address_space(3))) void *)dst, 16, (int)off, (int)soff, 0, 0);
 }
 
-// ---------------------------------------------------------------------------------------
-// the K loop of one pass (nch chunks): queue order of the loads is X0, R0 .. R(RING-2), X1,
-// R(RING-1) | per chunk c: X(c + 2), R(c + RING): waiting for an activation chunk never waits
-// for the weight chunks issued after it, so RING - 1 weight chunks stay in flight. Every load
-// is issued unconditionally (chunk indices clamped to the last chunk: a few repeated loads at
-// the end hit L2): with loads under branches the compiler cannot count them and waits for all.
-// ---------------------------------------------------------------------------------------
-template <int PREC, int RING, int NM, bool SC = false>
-__device__ __forceinline__ void k_loop(gu8 *const (&qp)[2], gu8 *const (&sp)[2], int nch, const uint16_t *srcrow,
-                                       uint16_t *s_a, DeqK dk, f32x16 (&d)[2][2], const int *ebrow = nullptr,
-                                       int emax = 0) {
+// row r of the pass's activation rows (UP: gathered, DOWN: consecutive pairs) that copy
+// instruction i of this wave reads, and the 16-byte block within the row
+template <int CK, int NM>
+__device__ __forceinline__ int astage_row(int i, int &blk) {
+    const int q = ((int)(threadIdx.x >> 6) + 4 * i) % AStage<CK>::total(NM), lane = threadIdx.x & 63;
+    const int r = q * AStage<CK>::RPI + lane / AStage<CK>::BPR;
+    blk = (lane % AStage<CK>::BPR) ^ AStage<CK>::swz(r);
+    return r;
+}
+
+// one chunk of MFMAs for a wave: CK / 16 steps x NM M tiles x 2 subtiles. Step m of lane half h
+// covers K h * CK / 2 + 8 m .. + 7 of the chunk, in A (LDS) and B (registers) alike. DOWN: h is
+// stored times 2^-eb per (pair, 32 columns); fx[mt][b] brings block b of the lane's half chunk to
+// the pair's largest exponent (exact unless the product is subnormal).
+template <int PREC, int NM, bool DOWN, int M = 0>
+__device__ __forceinline__ void mma_steps(const WChunk &w, const half2_t (&s2)[2], const uint16_t *ap, int v,
+                                          const half2_t (&fx)[NM][2], DeqK dk, f32x16 (*d)[2]) {
     constexpr int CK = GgPrec<PREC>::CK;
-    constexpr int ABUF = GG_TOK * GgChunk<CK>::LDA;
-    const int cl = nch - 1;
-    WChunk wr[RING];
-    uint4 xv[GgChunk<CK>::NV];
-    int xeb = 0;  // SC: the block exponent of the chunk in xv
-    auto xload = [&](int c) {
-        xs_load<CK>(srcrow, c, xv);
-        if constexpr (SC) xeb = ebrow[(c * CK + (threadIdx.x & 3) * GgChunk<CK>::VPT) / 32];
-    };
-    auto xstore = [&](uint16_t *dst) {
-        if constexpr (SC) xs_scale<CK>(xv, xeb, emax);
-        xs_store<CK>(xv, dst);
-    };
-    xload(0);
+    if constexpr (M < CK / 16) {
+        const f16x8 b0 = b_operand<PREC, M>(w.q[0], s2[0], dk);
+        const f16x8 b1 = b_operand<PREC, M>(w.q[1], s2[1], dk);
+        const uint16_t *am = ap + 8 * (v ^ M);
 #pragma unroll
-    for (int u = 0; u + 1 < RING; ++u) load_chunk<PREC>(wr[u], qp, sp, min(u, cl));
-    xstore(s_a);
-    xload(min(1, cl));
-    load_chunk<PREC>(wr[RING - 1], qp, sp, min(RING - 1, cl));
-    __syncthreads();
-#pragma unroll 1
-    for (int c0 = 0; c0 < nch; c0 += RING) {
-#pragma unroll
-        for (int u = 0; u < RING; ++u) {
-            const int c = c0 + u;
-            const int b = c & 1;
-            if (c < nch) mma_chunk<PREC, NM>(wr[u], s_a + b * ABUF, dk, d);
-            // unconditional: under a branch the compiler sinks the activation load of the previous
-            // step down to this store, and waiting for it then waits for every weight load too.
-            // The other buffer was last read before the previous barrier; a store past the last
-            // chunk is overwritten by the same thread in the next pass's prologue.
-            xstore(s_a + (b ^ 1) * ABUF);
-            xload(min(c + 2, cl));
-            load_chunk<PREC>(wr[u], qp, sp, min(c + RING, cl));
-            if (c < nch) __syncthreads();
+        for (int mt = 0; mt < NM; ++mt) {
+            f16x8 a = *reinterpret_cast<const f16x8 *>(am + mt * 32 * CK);
+            if constexpr (DOWN) {
+                const half2_t f = fx[mt][M / 4];
+                const f16x8 f8 = {f.x, f.x, f.x, f.x, f.x, f.x, f.x, f.x};
+                a = a * f8;
+            }
+            d[mt][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b0, d[mt][0], 0, 0, 0);
+            d[mt][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b1, d[mt][1], 0, 0, 0);
         }
+        mma_steps<PREC, NM, DOWN, M + 1>(w, s2, ap, v, fx, dk, d);
     }
 }
 
-// tile t -> (expert, block): the blocks of 8 consecutive experts interleave so that every tile of
-// one expert has the same t % 8 (workgroups go round-robin over the 8 XCDs)
-__device__ __forceinline__ bool tile_of(int t, int E, int NB, int &e, int &nb) {
-    const int eg = t / (8 * NB), r = t % (8 * NB);
-    e = eg * 8 + (r & 7);
+// ---------------------------------------------------------------------------------------
+// the K loop over chunks [0, nch) of a pass (NM M tiles). Weights: two chunks per wave in
+// registers (the second in flight while the first computes; with 3 workgroups per CU 48 KB of
+// them are in flight, and the stream needs about 20). Activations: S chunks in LDS, one barrier
+// per chunk. Queue order per chunk c: A(c + S - 1), [compute c], W(c + 2), scales(c + 2) on even c;
+// the wait before the barrier leaves what was issued after A(c + 1) outstanding: at least
+// (S - 2) activation chunks and one weight chunk. The last two chunks, which issue less, are
+// peeled (loads under a branch would make the compiler wait for all of them).
+// ---------------------------------------------------------------------------------------
+template <int N> __device__ __forceinline__ void wait_copies_and_sync() {
+    // this wave's copies older than the newest N vector memory operations have landed, its LDS
+    // reads are done; then every wave's
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+template <int PREC, int NMX, int S, int NM, bool DOWN, bool EVEN>
+__device__ __forceinline__ void k_loop(gu8 *qb, gu8 *sb, const uint32_t (&qo)[2], const uint32_t (&so)[2], int nch,
+                                       rsrc_t abuf, const uint32_t (&ao)[AStage<GgPrec<PREC>::CK>::per_wave(NM)],
+                                       uint16_t *s_a, const uint16_t *s_x, DeqK dk, f32x16 (*d)[2]) {
+    constexpr int CK = GgPrec<PREC>::CK;
+    constexpr int ABUF = 32 * NMX * CK;                // halves per stage
+    constexpr int NA = AStage<CK>::per_wave(NM);
+    constexpr int NW = 4;                              // weight loads per chunk
+    constexpr int WAIT = (S - 2) * NA + NW;
+    static_assert(S * ABUF * 2 <= 65536, "the copies' LDS offset is 16 bits");
+    const int cl = nch - 1;
+    const int lane = threadIdx.x & 63, i = lane & 31, h = lane >> 5, wave = uni((int)(threadIdx.x >> 6));
+    const uint16_t *ap = s_a + i * CK;
+    const int v = (h * (CK / 16)) ^ AStage<CK>::swz(i);
+    WChunk wr[2];
+    WScale sc, sn;
+    auto acopy = [&](int c, int buf) {
+#pragma unroll
+        for (int q = 0; q < NA; ++q)
+            lds_copy16(abuf, ao[q], (uint32_t)(c * CK * 2), s_a + buf * ABUF + ((wave + 4 * q) % AStage<CK>::total(NM)) * 512);
+    };
+    auto fence = [] {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto compute = [&](auto uc, int c, int buf) {
+        constexpr int U = decltype(uc)::value;
+        half2_t s2[2], fx[NM][2];
+        s2[0] = scale_of<PREC, U>(sc.s[0], h);
+        s2[1] = scale_of<PREC, U>(sc.s[1], h);
+        if constexpr (DOWN) {
+            // the factors of the 32-column blocks of this lane half's CK / 2 columns
+#pragma unroll
+            for (int mt = 0; mt < NM; ++mt)
+#pragma unroll
+                for (int b = 0; b < 2; ++b) {
+                    const int blk = (c * CK + h * (CK / 2)) / 32 + (CK == 128 ? b : 0);
+                    const uint32_t f = s_x[blk * (32 * NMX) + mt * 32 + i];
+                    fx[mt][b] = __builtin_bit_cast(half2_t, f | (f << 16));
+                }
+        }
+        mma_steps<PREC, NM, DOWN>(wr[U], s2, ap + buf * ABUF, v, fx, dk, d);
+    };
+    int buf = 0;  // stage of the current chunk
+    auto next = [&](int b) { return b + 1 == S ? 0 : b + 1; };
+    // a chunk with two more after it
+    auto step = [&](auto uc, int c) {
+        constexpr int U = decltype(uc)::value;
+        acopy(c + S - 1, S == 2 ? buf ^ 1 : (buf == 0 ? 2 : buf - 1));  // last read before the previous barrier
+        fence();
+        compute(uc, c, buf);
+        fence();
+        if constexpr (U == 0) load_scales<PREC, EVEN>(sn, sb, so, c + 2, cl);
+        else sc = sn;
+        fence();
+        load_chunk(wr[U], qb, qo, c + 2);
+        fence();
+        wait_copies_and_sync<WAIT>();
+        buf = next(buf);
+    };
+    // the last but one chunk
+    auto step_tail = [&](auto uc, int c) {
+        constexpr int U = decltype(uc)::value;
+        if constexpr (S == 2) acopy(c + 1, buf ^ 1);
+        fence();
+        compute(uc, c, buf);
+        fence();
+        if constexpr (U == 1) sc = sn;
+        wait_copies_and_sync<0>();
+        buf = next(buf);
+    };
+    // the caller's LDS tables are written, the previous pass's reads of the stages are done
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    load_scales<PREC, EVEN>(sc, sb, so, 0, cl);
+    load_chunk(wr[0], qb, qo, 0);
+    fence();
+    acopy(0, 0);
+    fence();
+    if constexpr (S == 3) acopy(min(1, cl), 1);
+    fence();
+    load_chunk(wr[1], qb, qo, min(1, cl));
+    fence();
+    wait_copies_and_sync<WAIT>();
+    if constexpr (EVEN) {
+        int c = 0;
+#pragma unroll 1
+        for (; c + 3 < nch; c += 2) {
+            step(IntC<0>{}, c);
+            step(IntC<1>{}, c + 1);
+        }
+        step_tail(IntC<0>{}, c);
+        compute(IntC<1>{}, c + 1, buf);
+    } else {  // an odd number of chunks
+        if (nch >= 3) {
+            int c = 0;
+#pragma unroll 1
+            for (; c + 4 < nch; c += 2) {
+                step(IntC<0>{}, c);
+                step(IntC<1>{}, c + 1);
+            }
+            step(IntC<0>{}, c);
+            step_tail(IntC<1>{}, c + 1);
+        }
+        compute(IntC<0>{}, cl, buf);
+    }
+    // no copy into LDS may be in flight past this point (one is only after a single-chunk loop)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+// Work units of the MFMA launches: an expert's pairs cut into passes of at most `tok` tokens (whole
+// 32-token tiles, as even as they go), in expert order: units[1 + u] = {expert, first pair (sorted
+// position), pairs, -}, units[0].x their number. A pass is a workgroup's work, so an expert with
+// many tokens (a shared expert has all of them) is spread over workgroups instead of being one
+// workgroup's chain of passes. At most min(E, NP) + NP / tok units. One workgroup of 256 threads;
+// offs(e): offsets[e].
+__host__ __device__ inline int gg_max_units(int E, int NP, int tok) { return min(E, NP) + NP / tok; }
+
+// exclusive scan of v over the 256 threads of a workgroup (s: 4 words of LDS), total in tot
+__device__ __forceinline__ int block_excl_scan256(int v, int *s, int &tot) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int incl = v;
+    for (int off = 1; off < 64; off <<= 1) {
+        const int o = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += o;
+    }
+    s[wave] = __builtin_amdgcn_readlane(incl, 63);
+    __syncthreads();
+    int base = 0;
+    tot = 0;
+    for (int w = 0; w < 4; ++w) {
+        if (w < wave) base += s[w];
+        tot += s[w];
+    }
+    __syncthreads();
+    return base + incl - v;
+}
+
+template <class F>
+__device__ __forceinline__ void gg_units(F offs, int E, int tok, int max_units, int4 *units, int *s_scan) {
+    int base = 0;
+    for (int e0 = 0; e0 < E; e0 += 256) {
+        const int e = e0 + (int)threadIdx.x;
+        const int p0 = e < E ? offs(e) : 0, ne = e < E ? offs(e + 1) - p0 : 0;
+        const int nt = (ne + 31) >> 5, np = (ne + tok - 1) / tok;
+        int tot;
+        const int u0 = base + block_excl_scan256(np, s_scan, tot);
+        int t0 = 0;
+        for (int m = 0; m < np; ++m) {
+            const int t1 = (nt * (m + 1) + np - 1) / np;  // tiles of passes 0 .. m
+            if (u0 + m < max_units) units[1 + u0 + m] = make_int4(e, p0 + 32 * t0, min(ne, 32 * t1) - 32 * t0, 0);
+            t0 = t1;
+        }
+        base += tot;
+    }
+    if (threadIdx.x == 0) units[0] = make_int4(min(base, max_units), 0, 0, 0);
+}
+
+// tile t -> (unit, block): the blocks of 8 consecutive units interleave so that every tile of one
+// unit has the same t % 8 (workgroups go round-robin over the 8 XCDs: a unit's activation rows are
+// re-read from one L2)
+__device__ __forceinline__ bool tile_of(int t, int U, int NB, int &u, int &nb) {
+    const int ug = t / (8 * NB), r = t % (8 * NB);
+    u = ug * 8 + (r & 7);
     nb = r >> 3;
-    return e < E;
+    return u < U;
 }
 
 // exponent e with max * 2^-e in [2^14, 2^15) (0 for 0, inf or nan)
@@ -337,21 +491,28 @@ __device__ __forceinline__ int row_exp(float m) {
     return (m > 0.f && m <= 3.0e38f) ? max(__builtin_amdgcn_frexp_expf(m) - 15, -100) : 0;
 }
 
-// bf16 activations, one wave per row: xe[r] = row_exp(max |x[r]|) and x16[r] = fp16(x[r] * 2^-xe[r])
-// (exact for bf16 values in range), 8 values per 16-byte load and store.
-// H is a multiple of 8.
 __device__ __forceinline__ float bf16_lo(uint32_t u) { return __uint_as_float(u << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t u) { return __uint_as_float(u & 0xffff0000u); }
 
-__global__ __launch_bounds__(256) void k_prep(const uint16_t *__restrict__ x, int T, int H, int *__restrict__ xe,
-                                              uint16_t *__restrict__ x16) {
-    const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (r >= T || x == nullptr) return;
-    const uint4 *src = reinterpret_cast<const uint4 *>(x + (size_t)r * H);
-    uint4 *dst = reinterpret_cast<uint4 *>(x16 + (size_t)r * H);
-    const int nv = H / 8;
+// 8 halves (a 16-byte block) from natural into operand order
+__device__ __forceinline__ uint4 operand_order(uint4 u) {
+    return make_uint4(lo_lo(u.x, u.z), hi_hi(u.x, u.z), lo_lo(u.y, u.w), hi_hi(u.y, u.w));
+}
+
+// one wave: a token's row of x (H values) as the MFMA tiles' operand, fp16 in operand order: fp16
+// activations as they are; bf16 times 2^-e, e = row_exp(max |x|) (exact for bf16 values in range).
+// H is a multiple of 8. Returns e.
+template <int DT>
+__device__ __forceinline__ int prep_row(const uint16_t *x, uint16_t *x16, int H) {
+    const int lane = threadIdx.x & 63;
+    const uint4 *src = reinterpret_cast<const uint4 *>(x);
+    uint4 *dst = reinterpret_cast<uint4 *>(x16);
+    if constexpr (DT == MOEHIP_DT_F16) {
+        for (int c = lane; c < H / 8; c += 64) dst[c] = operand_order(src[c]);
+        return 0;
+    }
     float m = 0.f;
-    for (int c = lane; c < nv; c += 64) {
+    for (int c = lane; c < H / 8; c += 64) {
         const uint4 v = src[c];
         const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
@@ -360,19 +521,30 @@ __global__ __launch_bounds__(256) void k_prep(const uint16_t *__restrict__ x, in
     m = wave_max(m);
     const int e = row_exp(m);
     const float sc = ldexpf(1.0f, -e);
-    for (int c = lane; c < nv; c += 64) {
+    for (int c = lane; c < H / 8; c += 64) {
         const uint4 v = src[c];
-        dst[c] = make_uint4(pack_h2(bf16_lo(v.x) * sc, bf16_hi(v.x) * sc), pack_h2(bf16_lo(v.y) * sc, bf16_hi(v.y) * sc),
-                            pack_h2(bf16_lo(v.z) * sc, bf16_hi(v.z) * sc), pack_h2(bf16_lo(v.w) * sc, bf16_hi(v.w) * sc));
+        dst[c] = operand_order(make_uint4(pack_h2(bf16_lo(v.x) * sc, bf16_hi(v.x) * sc), pack_h2(bf16_lo(v.y) * sc, bf16_hi(v.y) * sc),
+                                          pack_h2(bf16_lo(v.z) * sc, bf16_hi(v.z) * sc), pack_h2(bf16_lo(v.w) * sc, bf16_hi(v.w) * sc)));
     }
-    if (lane == 0) xe[r] = e;
+    return e;
 }
 
-// ---------------------------------------------------------------------------------------
-// up: tiles (expert, 128 h columns); wave w: h columns nb*128 + 32 w + (lane % 32), subtile 0 =
-// gate rows, subtile 1 = up rows. Writes h (pairs, I) fp32.
-// ---------------------------------------------------------------------------------------
-// x: fp16 activations (the caller's, or x16 with exponents xe for bf16 input; xe null = 0)
+// every token's row, and in workgroup 0 the work units (the others' rows hide it)
+template <int DT>
+__global__ __launch_bounds__(256) void k_prep(const uint16_t *__restrict__ x, int T, int H, int *__restrict__ xe,
+                                              uint16_t *__restrict__ x16, const int32_t *__restrict__ offsets, int E,
+                                              int tok, int max_units, int4 *__restrict__ units) {
+    __shared__ int s_scan[4];
+    if (blockIdx.x == 0) {
+        gg_units([&](int e) { return offsets[e]; }, E, tok, max_units, units, s_scan);
+        return;
+    }
+    const int r = (blockIdx.x - 1) * 4 + (threadIdx.x >> 6);
+    if (r >= T) return;
+    const int e = prep_row<DT>(x + (size_t)r * H, x16 + (size_t)r * H, H);
+    if ((threadIdx.x & 63) == 0) xe[r] = e;
+}
+
 // largest of a non-negative float over each 32-lane half of the wave, in every lane of the half
 // (every lane active), on the float's bits (their order is the values' for v >= 0; 0 is the
 // identity of the unsigned max, so each DPP move folds into its max): butterflies within rows of
@@ -387,69 +559,109 @@ __device__ __forceinline__ float half_max(float f) {
     return __uint_as_float(v);
 }
 
-template <int PREC>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_up(
-    const uint16_t *__restrict__ x, const int *__restrict__ xe, int H, int I, int k, int E,
-    const int32_t *__restrict__ offsets, const int32_t *__restrict__ sorted_pos, const int64_t *__restrict__ tab,
-    uint16_t *__restrict__ h16, int *__restrict__ hbe, DeqK dk) {
-    constexpr int CK = GgPrec<PREC>::CK;
-    __shared__ __align__(16) uint16_t s_a[2 * GG_TOK * GgChunk<CK>::LDA];
-    __shared__ int s_e[GG_TOK];
+// Passes of 32 * NMX tokens. NMX = 2 (S = 3 stages of activations): 64 accumulators per lane and 3
+// workgroups per CU, for few tokens per expert (bound by the weight stream). NMX = 4 (S = 2): the
+// conversion of a weight row, as much VALU work as the MFMAs of 64 tokens take, is shared by 128,
+// for many tokens per expert (bound by MFMA and the conversion).
+// A kernel's LDS is ONE object: with several the compiler tags each access with its object's alias
+// scope, and then waits for every activation copy in flight at each read of the stages (the waits
+// that are needed are in wait_copies_and_sync; the compiled loops hold no others).
+constexpr int GG_SEG = 1024;  // columns of h per factor table (32 blocks x the pass's tokens, 2 bytes each)
+template <int NA, int TOK> struct __align__(16) GgUpShared {
+    uint16_t a[NA];
+    int e[TOK];  // the tokens' exponents
+};
+template <int NA, int TOK> struct __align__(16) GgDownShared {
+    uint16_t a[NA];
+    uint16_t x[GG_SEG / 32 * TOK];  // [block of the segment][token]: 2^(eb - Emax)
+    float f[TOK];                   // w[pair] * 2^Emax
+};
+template <int NMX> struct GgPass {
+    static constexpr int TOK = 32 * NMX, S = NMX == 2 ? 3 : 2, WPE = NMX == 2 ? 3 : 2;
+};
+
+// ---------------------------------------------------------------------------------------
+// up: tiles (expert, 128 h columns); wave w: h columns nb*128 + 32 w + (lane % 32), subtile 0 =
+// gate rows, subtile 1 = up rows. x: fp16 in operand order with exponents xe (see prep_row). Writes
+// h16 (pairs, I): h = silu(gate) * up as fp16 times 2^-eb in operand order, hbe (pairs, I / 32): eb.
+// ---------------------------------------------------------------------------------------
+template <int PREC, int NMX>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GgPass<NMX>::WPE, GgPass<NMX>::WPE))) void k_gemm_up(
+    const uint16_t *__restrict__ x, uint32_t xbytes, const int *__restrict__ xe, int H, int I, int k, const int4 *__restrict__ units,
+    const int32_t *__restrict__ sorted_pos, const int64_t *__restrict__ tab, uint16_t *__restrict__ h16,
+    int8_t *__restrict__ hbe, DeqK dk) {
+    constexpr int CK = GgPrec<PREC>::CK, TOK = GgPass<NMX>::TOK, S = GgPass<NMX>::S;
+    __shared__ GgUpShared<S * TOK * CK, TOK> sh;
+    uint16_t *s_a = sh.a;
+    int *s_e = sh.e;
     const int NB = I / 128;
-    int e, nb;
-    if (!tile_of(blockIdx.x, E, NB, e, nb)) return;
-    const int p0 = offsets[e], ne = offsets[e + 1] - p0;
-    gu8 *qb = record_ptr(tab[4 * e + 0]);
-    gu8 *sb = record_ptr(tab[4 * e + 1]);
-    if (ne <= 0 || qb == nullptr) return;
+    int u, nb;
+    if (!tile_of(blockIdx.x, units[0].x, NB, u, nb)) return;
+    const int4 un = units[1 + u];
+    const int e = un.x, p0 = un.y, mn = un.z, nm = (mn + 31) / 32;
+    gu8 *qb = record_ptr(uni64(tab[4 * (size_t)e + 0]));
+    gu8 *sb = record_ptr(uni64(tab[4 * (size_t)e + 1]));
+    if (qb == nullptr) return;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, j = lane & 31, h = lane >> 5;
     const int col = nb * 128 + 32 * wave + j;
-    gu8 *qp[2], *sp[2];
-    gemm_rows<PREC>(qb, sb, col, H, h, qp[0], sp[0]);
-    gemm_rows<PREC>(qb, sb, I + col, H, h, qp[1], sp[1]);
+    uint32_t qo[2], so[2];
+    gemm_rows<PREC>(col, H, h, qo[0], so[0]);
+    gemm_rows<PREC>(I + col, H, h, qo[1], so[1]);
     const int nch = H / CK;
-    for (int m0 = 0; m0 < ne; m0 += GG_TOK) {
-        const int mn = min(GG_TOK, ne - m0), nm = (mn + 31) / 32;
-        const int stok = tid >> 2;
-        const bool sok = stok < mn;
-        const int xr = sok ? sorted_pos[p0 + m0 + stok] / k : 0;
-        const int ex = (sok && xe != nullptr) ? xe[xr] : 0;
-        if ((tid & 3) == 0) s_e[stok] = ex;
-        f32x16 d[2][2];
+    const rsrc_t xbuf = buffer_of(x, xbytes);
+    const int colp = (col & ~7) | ((col & 3) << 1) | ((col >> 2) & 1);  // operand order within 8
+    const int NB32 = I / 32;
+    const int32_t *sp = sorted_pos + p0;
+    if (tid < TOK) s_e[tid] = tid < mn ? xe[(uint32_t)sp[tid] / (uint32_t)k] : 0;
+    f32x16 d[NMX][2];
 #pragma unroll
-        for (int a = 0; a < 2; ++a)
+    for (int a = 0; a < NMX; ++a)
 #pragma unroll
-            for (int b = 0; b < 2; ++b) d[a][b] = f32x16{};
-        if (nm == 2) k_loop<PREC, 2, 2>(qp, sp, nch, x + (size_t)xr * H, s_a, dk, d);
-        else k_loop<PREC, 2, 1>(qp, sp, nch, x + (size_t)xr * H, s_a, dk, d);
-        // epilogue: h = silu(gate) * up (scaled back by the token's 2^e); per token the largest
-        // |h| of the wave's 32 columns (one half of the wave) sets the block exponent eb; h is
-        // stored fp16 times 2^-eb, eb beside it
-        // (branch-free first loop: the 16 lane reductions of a tile interleave)
-        const int NB32 = I / 32;
+        for (int b = 0; b < 2; ++b) d[a][b] = f32x16{};
+    auto loop = [&](auto nmc) {
+        constexpr int NM = decltype(nmc)::value, NA = AStage<CK>::per_wave(NM);
+        uint32_t ao[NA];
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt) {
-            if (mt >= nm) break;
+        for (int q = 0; q < NA; ++q) {
+            int blk;
+            const int r = astage_row<CK, NM>(q, blk);  // rows past the pass read its first row: never stored
+            ao[q] = (uint32_t)sp[r < mn ? r : 0] / (uint32_t)k * (uint32_t)(H * 2) + 16u * blk;
+        }
+        k_loop<PREC, NMX, S, NM, false, true>(qb, sb, qo, so, nch, xbuf, ao, s_a,
+                                              nullptr, dk, d);
+    };
+    if (nm == 1) loop(IntC<1>{});
+    else if (nm == 2) loop(IntC<2>{});
+    else if constexpr (NMX == 4) {
+        if (nm == 3) loop(IntC<3>{});
+        else loop(IntC<4>{});
+    }
+    // epilogue: h = silu(gate) * up (scaled back by the token's 2^e); per token the largest
+    // |h| of the wave's 32 columns (one half of the wave) sets the block exponent eb. SiLU from
+    // the hardware's exp2 and reciprocal (about 1 ulp of fp32 each; h is then rounded to fp16)
+    // (branch-free first loop: the 16 lane reductions of a tile interleave)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int tok = mt * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
-                const float f = ldexpf(1.0f, s_e[tok]);
-                const float hv = silu_mul(d[mt][0][r] * f, d[mt][1][r] * f);
-                d[mt][0][r] = hv;
-                d[mt][1][r] = half_max(fabsf(hv));
-            }
+    for (int mt = 0; mt < NMX; ++mt) {
+        if (mt >= nm) break;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int tok = mt * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
-                const int eb = row_exp(d[mt][1][r]);
-                if (tok < mn) {
-                    const size_t p = (size_t)(p0 + m0 + tok);
-                    h16[p * I + col] = f32_to_f16_rne(d[mt][0][r] * ldexpf(1.0f, -eb));
-                    if (j == 0) hbe[p * NB32 + (col >> 5)] = eb;
-                }
+        for (int r = 0; r < 16; ++r) {
+            const int tok = mt * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
+            const int ex = s_e[tok];
+            const float hv = silu_mul_fast(__builtin_amdgcn_ldexpf(d[mt][0][r], ex), __builtin_amdgcn_ldexpf(d[mt][1][r], ex));
+            d[mt][0][r] = hv;
+            d[mt][1][r] = half_max(fabsf(hv));
+        }
+        uint16_t *hr = h16 + (size_t)(p0 + mt * 32 + 4 * h) * I + colp;
+        int8_t *er = hbe + (size_t)(p0 + mt * 32 + 4 * h) * NB32 + (col >> 5);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int tr = 8 * (r >> 2) + (r & 3);
+            const int eb = row_exp(d[mt][1][r]);
+            if (mt * 32 + 4 * h + tr < mn) {
+                hr[(uint32_t)(tr * I)] = f32_to_f16_rne(__builtin_amdgcn_ldexpf(d[mt][0][r], -eb));
+                if (j == 0) er[(uint32_t)(tr * NB32)] = (int8_t)eb;
             }
         }
-        __syncthreads();  // s_e of the next pass
     }
 }
 
@@ -888,74 +1100,106 @@ __global__ __launch_bounds__(256) void k_gemv_down2(const float *__restrict__ hb
 // ---------------------------------------------------------------------------------------
 // down: tiles (expert, 256 output rows); wave w: rows nb*256 + 64 w + 32 t + (lane % 32).
 // y[pair, row] = w[pair] * (down_row . h_pair); h is read as the up tiles left it (fp16 times
-// 2^-eb per 32 columns) and rescaled to the pair's largest exponent Emax while staged
+// 2^-eb per 32 columns) and brought to the pair's largest exponent Emax as the A operands are
+// read from LDS, by the factors 2^(eb - Emax) of a table per segment of GG_SEG columns
 // ---------------------------------------------------------------------------------------
-template <int PREC>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_down(
-    const uint16_t *__restrict__ h16, const int *__restrict__ hbe, int H, int I, int E,
-    const int32_t *__restrict__ offsets, const int32_t *__restrict__ sorted_pos, const int64_t *__restrict__ tab,
-    const float *__restrict__ w, float *__restrict__ y, DeqK dk, int zero_missing) {
-    constexpr int CK = GgPrec<PREC>::CK;
-    __shared__ __align__(16) uint16_t s_a[2 * GG_TOK * GgChunk<CK>::LDA];
-    __shared__ float s_f[GG_TOK];  // w[pair] * 2^Emax
+// int4 rows at 64-token passes: 3 waves per SIMD spill (54 us against 48 with 2 at d_model 2048, d_ff
+// 768, 128 experts, 512 tokens); the other kinds fit (fp8 at 512 experts: 127 us with 3, 134 with 2)
+constexpr int gg_down_wpe(int prec, int nmx) { return nmx == 2 && prec != MOEHIP_PREC_INT4 ? 3 : 2; }
+template <int PREC, int NMX, bool EVEN>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(gg_down_wpe(PREC, NMX), gg_down_wpe(PREC, NMX)))) void k_gemm_down(
+    const uint16_t *__restrict__ h16, const int8_t *__restrict__ hbe, int H, int I, const int4 *__restrict__ units,
+    const int32_t *__restrict__ sorted_pos, const int64_t *__restrict__ tab, const float *__restrict__ w,
+    float *__restrict__ y, DeqK dk, int zero_missing) {
+    constexpr int CK = GgPrec<PREC>::CK, TOK = GgPass<NMX>::TOK, S = GgPass<NMX>::S, TPT = 256 / TOK;
+    __shared__ GgDownShared<S * TOK * CK, TOK> sh;
+    uint16_t *s_a = sh.a, *s_x = sh.x;
+    float *s_f = sh.f;
     const int NB = H / GG_ROWS;
-    int e, nb;
-    if (!tile_of(blockIdx.x, E, NB, e, nb)) return;
-    const int p0 = offsets[e], ne = offsets[e + 1] - p0;
-    if (ne <= 0) return;
+    int u, nb;
+    if (!tile_of(blockIdx.x, units[0].x, NB, u, nb)) return;
+    const int4 un = units[1 + u];
+    const int e = un.x, p0 = un.y, mn = un.z, nm = (mn + 31) / 32;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, j = lane & 31, h = lane >> 5;
-    gu8 *qb = record_ptr(tab[4 * e + 2]);
-    gu8 *sb = record_ptr(tab[4 * e + 3]);
+    gu8 *qb = record_ptr(uni64(tab[4 * (size_t)e + 2]));
+    gu8 *sb = record_ptr(uni64(tab[4 * (size_t)e + 3]));
     const int row0 = nb * GG_ROWS + 64 * wave + j;
     if (qb == nullptr) {  // expert not resident (single-table launches): its pairs contribute nothing
         if (zero_missing)
-            for (int i = tid; i < ne * GG_ROWS; i += 256)
+            for (int i = tid; i < mn * GG_ROWS; i += 256)
                 y[(size_t)(p0 + i / GG_ROWS) * H + nb * GG_ROWS + i % GG_ROWS] = 0.f;
         return;
     }
-    gu8 *qp[2], *sp[2];
-    gemm_rows<PREC>(qb, sb, row0, I, h, qp[0], sp[0]);
-    gemm_rows<PREC>(qb, sb, row0 + 32, I, h, qp[1], sp[1]);
-    const int nch = I / CK;
-    for (int m0 = 0; m0 < ne; m0 += GG_TOK) {
-        const int mn = min(GG_TOK, ne - m0), nm = (mn + 31) / 32;
-        const int stok = tid >> 2;
-        const bool sok = stok < mn;
-        const size_t pr = (size_t)(p0 + m0 + (sok ? stok : 0));
-        // the pair's largest block exponent: the 4 staging threads of the pair take every 4th
-        // block (independent loads, issued together), then the largest over the 4 (DPP)
-        const int NB32 = I / 32;
-        const int *ebrow = hbe + pr * NB32;
-        int emax = -1000;
-        for (int i0 = tid & 3; i0 < NB32; i0 += 32) {
+    uint32_t qo[2], so[2];
+    gemm_rows<PREC>(row0, I, h, qo[0], so[0]);
+    gemm_rows<PREC>(row0 + 32, I, h, qo[1], so[1]);
+    const int stok = tid / TPT, part = tid % TPT;
+    const bool sok = stok < mn;
+    const size_t pr = (size_t)(p0 + (sok ? stok : 0));
+    // the pair's largest block exponent: the TPT threads of the pair take every TPT-th dword (4
+    // blocks), then the largest over them (DPP)
+    const int ND = I / 128;
+    const uint32_t *eb4 = reinterpret_cast<const uint32_t *>(hbe + pr * (I / 32));
+    int emax = -1000;
+    for (int i0 = part; i0 < ND; i0 += TPT) {
+        const int v = (int)eb4[i0];
+        emax = max(max(emax, max((v << 24) >> 24, (v << 16) >> 24)), max((v << 8) >> 24, v >> 24));
+    }
+    emax = max(emax, dpp_i<0xB1>(emax));
+    if constexpr (TPT == 4) emax = max(emax, dpp_i<0x4E>(emax));
+    if (part == 0) s_f[stok] = sok ? w[sorted_pos[pr]] * ldexpf(1.0f, emax) : 0.f;
+    f32x16 d[NMX][2];
 #pragma unroll
-            for (int i = 0; i < 8; ++i)
-                if (i0 + 4 * i < NB32) emax = max(emax, ebrow[i0 + 4 * i]);
+    for (int a = 0; a < NMX; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) d[a][b] = f32x16{};
+    auto loop = [&](auto nmc) {
+        constexpr int NM = decltype(nmc)::value, NA = AStage<CK>::per_wave(NM);
+        uint32_t ao[NA];
+#pragma unroll
+        for (int q = 0; q < NA; ++q) {
+            int blk;
+            const int r = astage_row<CK, NM>(q, blk);
+            ao[q] = (uint32_t)(r < mn ? r : 0) * (uint32_t)(I * 2) + 16u * blk;
         }
-        emax = max(emax, dpp_i<0xB1>(emax));
-        emax = max(emax, dpp_i<0x4E>(emax));
-        if ((tid & 3) == 0) s_f[stok] = sok ? w[sorted_pos[pr]] * ldexpf(1.0f, emax) : 0.f;
-        f32x16 d[2][2];
+#pragma unroll 1
+        for (int k0 = 0; k0 < I; k0 += GG_SEG) {
+            const int kn = min(GG_SEG, I - k0);
+            if (k0 != 0) __syncthreads();  // the previous segment's factors have been read
+            for (int i0 = part; i0 < kn / 128; i0 += TPT) {
+                const int v = (int)eb4[k0 / 128 + i0];
+                const int eb[4] = {(v << 24) >> 24, (v << 16) >> 24, (v << 8) >> 24, v >> 24};
 #pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int b = 0; b < 2; ++b) d[a][b] = f32x16{};
-        if (nm == 2) k_loop<PREC, 2, 2, true>(qp, sp, nch, h16 + pr * I, s_a, dk, d, ebrow, emax);
-        else k_loop<PREC, 2, 1, true>(qp, sp, nch, h16 + pr * I, s_a, dk, d, ebrow, emax);
-#pragma unroll
-        for (int mt = 0; mt < 2; ++mt) {
-            if (mt >= nm) break;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int tok = mt * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
-                if (tok >= mn) continue;
-                const size_t p = (size_t)(p0 + m0 + tok);
-                const float f = s_f[tok];
-                y[p * H + row0] = f * d[mt][0][r];
-                y[p * H + row0 + 32] = f * d[mt][1][r];
+                for (int q = 0; q < 4; ++q) s_x[(4 * i0 + q) * TOK + stok] = (uint16_t)pow2_h(eb[q] - emax);
             }
+            // (the K loop starts with a barrier)
+            gu8 *qs = qb + (size_t)k0 * GgPrec<PREC>::BITS / 8;
+            gu8 *ss = sb;
+            if constexpr (PREC == MOEHIP_PREC_INT4 || PREC == MOEHIP_PREC_INT8) ss += k0 / GG_KG * 2;
+            else if constexpr (PREC == MOEHIP_PREC_FP8) ss += k0 / 128 * 4;
+            // (the pass's rows from column k0 on)
+            const rsrc_t hbuf = buffer_of(h16 + (size_t)p0 * I + k0, (uint32_t)(mn * I - k0) * 2u);
+            k_loop<PREC, NMX, S, NM, true, EVEN>(qs, ss, qo, so, kn / CK, hbuf, ao, s_a, s_x, dk, d);
         }
-        __syncthreads();  // s_f of the next pass
+    };
+    if (nm == 1) loop(IntC<1>{});
+    else if (nm == 2) loop(IntC<2>{});
+    else if constexpr (NMX == 4) {
+        if (nm == 3) loop(IntC<3>{});
+        else loop(IntC<4>{});
+    }
+#pragma unroll
+    for (int mt = 0; mt < NMX; ++mt) {
+        if (mt >= nm) break;
+        float *yr = y + (size_t)(p0 + mt * 32 + 4 * h) * H + row0;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int tr = 8 * (r >> 2) + (r & 3);
+            if (mt * 32 + 4 * h + tr >= mn) continue;
+            const float f = s_f[mt * 32 + 4 * h + tr];
+            yr[(uint32_t)(tr * H)] = f * d[mt][0][r];
+            yr[(uint32_t)(tr * H) + 32] = f * d[mt][1][r];
+        }
     }
 }
 
@@ -1156,7 +1400,7 @@ __device__ __forceinline__ void stage_store(const XStage<CK, NT> &s, int emax, u
             u.z = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, u.z) * f2);
             u.w = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, u.w) * f2);
         }
-        dst[m] = make_uint4(lo_lo(u.x, u.z), hi_hi(u.x, u.z), lo_lo(u.y, u.w), hi_hi(u.y, u.w));
+        dst[m] = DOWN ? operand_order(u) : u;  // (x comes in operand order)
     }
 }
 
@@ -1230,11 +1474,13 @@ __device__ __forceinline__ void mma_chunk16(const WChunk16 &w, const uint16_t *s
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
             const uint4 qq[2] = {w.q[t], w.q[t]};
+            const uint32_t sw = PREC == MOEHIP_PREC_FP8 ? f32_to_f16_rne(__uint_as_float(w.s[t]) * 256.0f) : w.s[t] & 0xffffu;
+            const half2_t s2 = __builtin_bit_cast(half2_t, sw | (sw << 16));
             switch (M) {  // b_operand takes the step as a template argument
-                case 0: b[t] = b_operand<PREC, 0>(qq, w.s[t], dk); break;
-                case 1: b[t] = b_operand<PREC, (S > 1 ? 1 : 0)>(qq, w.s[t], dk); break;
-                case 2: b[t] = b_operand<PREC, (S > 2 ? 2 : 0)>(qq, w.s[t], dk); break;
-                default: b[t] = b_operand<PREC, (S > 3 ? 3 : 0)>(qq, w.s[t], dk); break;
+                case 0: b[t] = b_operand<PREC, 0>(qq, s2, dk); break;
+                case 1: b[t] = b_operand<PREC, (S > 1 ? 1 : 0)>(qq, s2, dk); break;
+                case 2: b[t] = b_operand<PREC, (S > 2 ? 2 : 0)>(qq, s2, dk); break;
+                default: b[t] = b_operand<PREC, (S > 3 ? 3 : 0)>(qq, s2, dk); break;
             }
         }
 #pragma unroll
@@ -1612,32 +1858,12 @@ constexpr int RP_STRIDE = 32;   // words between two experts' counters: a 128-by
                                 // atomics on counters sharing lines queue on one memory channel)
 constexpr int RP_DONE = RP_MAXE * RP_STRIDE;  // words of the counter area
 
-// exclusive scan of v over the 256 threads of a workgroup (s: 4 words of LDS), total in tot
-__device__ __forceinline__ int block_excl_scan256(int v, int *s, int &tot) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int incl = v;
-    for (int off = 1; off < 64; off <<= 1) {
-        const int o = __shfl_up(incl, off, 64);
-        if (lane >= off) incl += o;
-    }
-    s[wave] = __builtin_amdgcn_readlane(incl, 63);
-    __syncthreads();
-    int base = 0;
-    tot = 0;
-    for (int w = 0; w < 4; ++w) {
-        if (w < wave) base += s[w];
-        tot += s[w];
-    }
-    __syncthreads();
-    return base + incl - v;
-}
-
 template <int DT>
 __global__ __launch_bounds__(256) void k_route_post(const void *__restrict__ logits, const uint16_t *__restrict__ x,
                                                     int T, int H, int E, int k, int renorm, int64_t *__restrict__ idx,
                                                     void *__restrict__ wout, float *__restrict__ w32,
                                                     int *__restrict__ cnt, int *__restrict__ bucket,
-                                                    int *__restrict__ xe, uint16_t *__restrict__ x16, int prep) {
+                                                    int *__restrict__ xe, uint16_t *__restrict__ x16) {
     __shared__ float s_p[4][32];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int t = blockIdx.x * 4 + wave;
@@ -1655,26 +1881,8 @@ __global__ __launch_bounds__(256) void k_route_post(const void *__restrict__ log
             // test keeps a corrupted counter from writing past the bucket
             if (r < T) bucket[(size_t)myc * T + r] = (int)q;
         }
-        if (prep) {  // the token's row: fp16 with max |x| in [2^14, 2^15) (k_prep's rule)
-            const uint4 *src = reinterpret_cast<const uint4 *>(x + (size_t)t * H);
-            uint4 *dst = reinterpret_cast<uint4 *>(x16 + (size_t)t * H);
-            float m = 0.f;
-            for (int c = lane; c < H / 8; c += 64) {
-                const uint4 v = src[c];
-                const uint32_t wd[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                for (int i = 0; i < 4; ++i) m = fmaxf(m, fmaxf(fabsf(bf16_lo(wd[i])), fabsf(bf16_hi(wd[i]))));
-            }
-            m = wave_max(m);
-            const int e = row_exp(m);
-            const float sc = ldexpf(1.0f, -e);
-            for (int c = lane; c < H / 8; c += 64) {
-                const uint4 v = src[c];
-                dst[c] = make_uint4(pack_h2(bf16_lo(v.x) * sc, bf16_hi(v.x) * sc), pack_h2(bf16_lo(v.y) * sc, bf16_hi(v.y) * sc),
-                                    pack_h2(bf16_lo(v.z) * sc, bf16_hi(v.z) * sc), pack_h2(bf16_lo(v.w) * sc, bf16_hi(v.w) * sc));
-            }
-            if (lane == 0) xe[t] = e;
-        }
+        const int e = prep_row<DT>(x + (size_t)t * H, x16 + (size_t)t * H, H);
+        if (lane == 0) xe[t] = e;
     }
 }
 
@@ -1684,7 +1892,8 @@ __global__ __launch_bounds__(256) void k_route_post(const void *__restrict__ log
 __global__ __launch_bounds__(256) void k_route_place(const int *__restrict__ cnt, const int *__restrict__ bucket,
                                                      int T, int k, int E, int32_t *__restrict__ counts,
                                                      int32_t *__restrict__ offsets, int32_t *__restrict__ sorted_pos,
-                                                     int32_t *__restrict__ rank) {
+                                                     int32_t *__restrict__ rank, int tok, int max_units,
+                                                     int4 *__restrict__ units) {
     __shared__ int s_off[RP_MAXE + 1];
     __shared__ int s_scan[4];
     int c4[4], loc = 0;
@@ -1713,6 +1922,10 @@ __global__ __launch_bounds__(256) void k_route_place(const int *__restrict__ cnt
         if (blockIdx.x == 0) offsets[E] = total;
     }
     __syncthreads();
+    if (blockIdx.x == gridDim.x - 1) {  // a workgroup of its own: the work units
+        gg_units([&](int e) { return s_off[e]; }, E, tok, max_units, units, s_scan);
+        return;
+    }
     const int q = blockIdx.x * 256 + threadIdx.x;
     if (q >= T * k) return;
     if (q >= total) {
@@ -1732,7 +1945,7 @@ __global__ __launch_bounds__(256) void k_route_place(const int *__restrict__ cnt
 }
 
 struct GgLayout {
-    size_t xe, x16, h, h16, y, items, hbe, plan, list, pairs, dummy, total;
+    size_t xe, x16, h, h16, y, items, units, hbe, plan, list, pairs, dummy, total;
     int lmax;
 };
 static GgLayout gg_layout(int T, int k, int H, int I) {
@@ -1752,6 +1965,8 @@ static GgLayout gg_layout(int T, int k, int H, int I) {
     off = al(off + NP * H * 4);
     L.items = off;  // one work list per record precision
     off = al(off + (size_t)GV_MAXP * (NP + 1) * 4);
+    L.units = off;  // (per 64 tokens: the longer of the two lists; at most one unit per pair)
+    off = al(off + ((size_t)gg_max_units((int)NP, (int)NP, 64) + 1) * 16);
     // the block exponents of h (one per pair and 32 columns; the persistent FFN's one per 128),
     // the persistent FFN's plan words and tile queues
     const int NBU = I / 128, NBD = H / GG_ROWS;
@@ -1779,18 +1994,39 @@ extern "C" size_t moehip_grouped_gemm_workspace_bytes(int T, int k, int H, int I
     return gg_layout(T, k, H, I).total;
 }
 
+// Tokens per pass of the MFMA launches, from the mean pairs per expert (the counts themselves are on
+// the device; an expert of any size is correct in either).
+static int gg_tokens(int NP, int E) { return NP >= 48 * (int64_t)E ? 128 : 64; }
+
 template <int PREC>
-static void launch_up(dim3 g, hipStream_t st, const uint16_t *x, const int *xe, int H, int I, int k, int E,
-                      const int32_t *offsets, const int32_t *sorted_pos, const int64_t *tab, uint16_t *h16, int *hbe,
+static void launch_up(int tok, int MU, hipStream_t st, const uint16_t *x, uint32_t xbytes, const int *xe, int H, int I, int k,
+                      const int4 *units, const int32_t *sorted_pos, const int64_t *tab, uint16_t *h16, int8_t *hbe,
                       DeqK dk) {
-    hipLaunchKernelGGL((k_gemm_up<PREC>), g, dim3(256), 0, st, x, xe, H, I, k, E, offsets, sorted_pos, tab, h16, hbe, dk);
+    const dim3 g((MU + 7) / 8 * 8 * (I / 128));
+    if (tok == 128) hipLaunchKernelGGL((k_gemm_up<PREC, 4>), g, dim3(256), 0, st, x, xbytes, xe, H, I, k, units, sorted_pos, tab, h16, hbe, dk);
+    else hipLaunchKernelGGL((k_gemm_up<PREC, 2>), g, dim3(256), 0, st, x, xbytes, xe, H, I, k, units, sorted_pos, tab, h16, hbe, dk);
+}
+template <int PREC, bool EVEN>
+static void launch_down_e(int tok, int MU, hipStream_t st, const uint16_t *h16, const int8_t *hbe, int H, int I,
+                          const int4 *units, const int32_t *sorted_pos, const int64_t *tab, const float *w, float *y,
+                          DeqK dk, int zero_missing) {
+    const dim3 g((MU + 7) / 8 * 8 * (H / GG_ROWS));
+    if (tok == 128)
+        hipLaunchKernelGGL((k_gemm_down<PREC, 4, EVEN>), g, dim3(256), 0, st, h16, hbe, H, I, units, sorted_pos, tab, w, y, dk, zero_missing);
+    else
+        hipLaunchKernelGGL((k_gemm_down<PREC, 2, EVEN>), g, dim3(256), 0, st, h16, hbe, H, I, units, sorted_pos, tab, w, y, dk, zero_missing);
 }
 template <int PREC>
-static void launch_down(dim3 g, hipStream_t st, const uint16_t *h16, const int *hbe, int H, int I, int E,
-                        const int32_t *offsets, const int32_t *sorted_pos, const int64_t *tab, const float *w, float *y,
+static void launch_down(int tok, int MU, hipStream_t st, const uint16_t *h16, const int8_t *hbe, int H, int I,
+                        const int4 *units, const int32_t *sorted_pos, const int64_t *tab, const float *w, float *y,
                         DeqK dk, int zero_missing) {
-    hipLaunchKernelGGL((k_gemm_down<PREC>), g, dim3(256), 0, st, h16, hbe, H, I, E, offsets, sorted_pos, tab, w, y, dk,
-                       zero_missing);
+    if constexpr (PREC == MOEHIP_PREC_INT4) {  // the other kinds have an even number of chunks for any I
+        if (I % 256 != 0) {
+            launch_down_e<PREC, false>(tok, MU, st, h16, hbe, H, I, units, sorted_pos, tab, w, y, dk, zero_missing);
+            return;
+        }
+    }
+    launch_down_e<PREC, true>(tok, MU, st, h16, hbe, H, I, units, sorted_pos, tab, w, y, dk, zero_missing);
 }
 
 // the persistent FFN of one record table: plan, then one workgroup per CU slot (at most)
@@ -2015,24 +2251,29 @@ static int gg_run(int P, const int *precs, const int64_t *tabs, const void *x, i
     float *y = reinterpret_cast<float *>(wsb + L.y);
     const int NP = T * k;
     hipStream_t st = as_stream(stream);
-    const int E8 = (E + 7) / 8 * 8;
-    const dim3 gu(E8 * (I / 128)), gd(E8 * (H / GG_ROWS));
+    const int tok = gg_tokens(NP, E), MU = gg_max_units(E, NP, tok);
+    int4 *units = reinterpret_cast<int4 *>(wsb + L.units);
     const uint16_t *xs = reinterpret_cast<const uint16_t *>(x);
     uint16_t *x16 = reinterpret_cast<uint16_t *>(wsb + L.x16);
     const DeqK dk = {0x000F000Fu, 0x64006400u};
     const bool bf = xdtype == MOEHIP_DT_BF16;
-    const uint16_t *xa = bf ? x16 : xs;
-    const int *xea = bf ? xe : nullptr;
-    // bf16 activations: fp16 with a per-token power of two for the MFMA tiles; the GEMVs read
-    // the bf16 rows themselves and scale each chunk
-    if (bf && !gemv && !x16_ready) hipLaunchKernelGGL(k_prep, dim3((T + 3) / 4), dim3(256), 0, st, xs, T, H, xe, x16);
+    // the MFMA tiles' operand (fp16 in operand order, bf16 with a per-token power of two) and their
+    // work units; the GEMVs read x itself (bf16: each chunk scaled)
+    if (!gemv && !x16_ready) {
+        if (bf) hipLaunchKernelGGL((k_prep<MOEHIP_DT_BF16>), dim3((T + 3) / 4 + 1), dim3(256), 0, st, xs, T, H, xe, x16, offsets, E, tok, MU, units);
+        else hipLaunchKernelGGL((k_prep<MOEHIP_DT_F16>), dim3((T + 3) / 4 + 1), dim3(256), 0, st, xs, T, H, xe, x16, offsets, E, tok, MU, units);
+    }
     // MFMA tiles: the separate up / h / down launches below, or (MOEHIP_GEMM_FUSED set, where
-    // workgroups are dealt to the XCDs round robin) the persistent FFN, one launch per record table
-    const bool fused = !gemv && xcd_dispatch_ok() && getenv("MOEHIP_GEMM_FUSED") != nullptr;
+    // workgroups are dealt to the XCDs round robin) the persistent FFN, one launch per record table.
+    // The separate launches address x16 and the routed rows by 32-bit buffer offsets: 4 GB of x16 or
+    // more (a million tokens at d_model 2048) go through the persistent FFN's 64-bit addresses
+    const bool wide = (uint64_t)T * H * 2 >= (1ull << 32);
+    MOEHIP_REQUIRE(gemv || !wide || xcd_dispatch_ok(), "grouped_gemm: %d tokens need a device set up by moehip_device_check", T);
+    const bool fused = !gemv && xcd_dispatch_ok() && (wide || getenv("MOEHIP_GEMM_FUSED") != nullptr);
     if (fused) {
         FfnArgs fa{};
-        fa.x = xa;
-        fa.xe = xea;
+        fa.x = x16;
+        fa.xe = xe;
         fa.H = H;
         fa.I = I;
         fa.k = k;
@@ -2071,22 +2312,22 @@ static int gg_run(int P, const int *precs, const int64_t *tabs, const void *x, i
     if (items_in != nullptr) items = const_cast<int32_t *>(items_in);
     // a two-precision store: both precisions in one up and one down launch where the pair is instantiated
     const bool two = gemv && P == 2 &&
-                     launch_gv2(precs, bf ? 2 : 1, items, NP, st, bf ? xs : xa, bf ? nullptr : xea, H, I, k, offsets,
+                     launch_gv2(precs, bf ? 2 : 1, items, NP, st, xs, nullptr, H, I, k, offsets,
                                 sorted_pos, tabs, E, hb, nullptr, dk);
     for (int p = 0; p < P && gemv && !two; ++p)
-        launch_gv_prec(precs[p], bf ? 2 : 1, items + (size_t)p * (NP + 1), NP, st, bf ? xs : xa, bf ? nullptr : xea, H, I, k, offsets, sorted_pos, tabs + (size_t)p * E * 4, hb, nullptr,
+        launch_gv_prec(precs[p], bf ? 2 : 1, items + (size_t)p * (NP + 1), NP, st, xs, nullptr, H, I, k, offsets, sorted_pos, tabs + (size_t)p * E * 4, hb, nullptr,
                        dk);
     // the MFMA up tiles write h as fp16 with a power of two per (pair, 32 columns); the GEMVs fp32
     uint16_t *h16 = reinterpret_cast<uint16_t *>(wsb + L.h16);
-    int *hbe = reinterpret_cast<int *>(wsb + L.hbe);
+    int8_t *hbe = reinterpret_cast<int8_t *>(wsb + L.hbe);
     for (int p = 0; p < P && !gemv && !fused; ++p) {
         const int64_t *tab = tabs + (size_t)p * E * 4;
         switch (precs[p]) {
-            case MOEHIP_PREC_INT4: launch_up<MOEHIP_PREC_INT4>(gu, st, xa, xea, H, I, k, E, offsets, sorted_pos, tab, h16, hbe, dk); break;
-            case MOEHIP_PREC_INT8: launch_up<MOEHIP_PREC_INT8>(gu, st, xa, xea, H, I, k, E, offsets, sorted_pos, tab, h16, hbe, dk); break;
-            case MOEHIP_PREC_FP8: launch_up<MOEHIP_PREC_FP8>(gu, st, xa, xea, H, I, k, E, offsets, sorted_pos, tab, h16, hbe, dk); break;
-            case MOEHIP_PREC_F16: launch_up<MOEHIP_PREC_F16>(gu, st, xa, xea, H, I, k, E, offsets, sorted_pos, tab, h16, hbe, dk); break;
-            default: launch_up<MOEHIP_PREC_BF16>(gu, st, xa, xea, H, I, k, E, offsets, sorted_pos, tab, h16, hbe, dk); break;
+            case MOEHIP_PREC_INT4: launch_up<MOEHIP_PREC_INT4>(tok, MU, st, x16, (uint32_t)((size_t)T * H * 2), xe, H, I, k, units, sorted_pos, tab, h16, hbe, dk); break;
+            case MOEHIP_PREC_INT8: launch_up<MOEHIP_PREC_INT8>(tok, MU, st, x16, (uint32_t)((size_t)T * H * 2), xe, H, I, k, units, sorted_pos, tab, h16, hbe, dk); break;
+            case MOEHIP_PREC_FP8: launch_up<MOEHIP_PREC_FP8>(tok, MU, st, x16, (uint32_t)((size_t)T * H * 2), xe, H, I, k, units, sorted_pos, tab, h16, hbe, dk); break;
+            case MOEHIP_PREC_F16: launch_up<MOEHIP_PREC_F16>(tok, MU, st, x16, (uint32_t)((size_t)T * H * 2), xe, H, I, k, units, sorted_pos, tab, h16, hbe, dk); break;
+            default: launch_up<MOEHIP_PREC_BF16>(tok, MU, st, x16, (uint32_t)((size_t)T * H * 2), xe, H, I, k, units, sorted_pos, tab, h16, hbe, dk); break;
         }
     }
     if (two) launch_gv2(precs, 0, items, NP, st, hb, nullptr, H, I, k, offsets, sorted_pos, tabs, E, y, w, dk);
@@ -2097,11 +2338,11 @@ static int gg_run(int P, const int *precs, const int64_t *tabs, const void *x, i
         const int64_t *tab = tabs + (size_t)p * E * 4;
         const int zm = zero_missing && P == 1;
         switch (precs[p]) {
-            case MOEHIP_PREC_INT4: launch_down<MOEHIP_PREC_INT4>(gd, st, h16, hbe, H, I, E, offsets, sorted_pos, tab, w, y, dk, zm); break;
-            case MOEHIP_PREC_INT8: launch_down<MOEHIP_PREC_INT8>(gd, st, h16, hbe, H, I, E, offsets, sorted_pos, tab, w, y, dk, zm); break;
-            case MOEHIP_PREC_FP8: launch_down<MOEHIP_PREC_FP8>(gd, st, h16, hbe, H, I, E, offsets, sorted_pos, tab, w, y, dk, zm); break;
-            case MOEHIP_PREC_F16: launch_down<MOEHIP_PREC_F16>(gd, st, h16, hbe, H, I, E, offsets, sorted_pos, tab, w, y, dk, zm); break;
-            default: launch_down<MOEHIP_PREC_BF16>(gd, st, h16, hbe, H, I, E, offsets, sorted_pos, tab, w, y, dk, zm); break;
+            case MOEHIP_PREC_INT4: launch_down<MOEHIP_PREC_INT4>(tok, MU, st, h16, hbe, H, I, units, sorted_pos, tab, w, y, dk, zm); break;
+            case MOEHIP_PREC_INT8: launch_down<MOEHIP_PREC_INT8>(tok, MU, st, h16, hbe, H, I, units, sorted_pos, tab, w, y, dk, zm); break;
+            case MOEHIP_PREC_FP8: launch_down<MOEHIP_PREC_FP8>(tok, MU, st, h16, hbe, H, I, units, sorted_pos, tab, w, y, dk, zm); break;
+            case MOEHIP_PREC_F16: launch_down<MOEHIP_PREC_F16>(tok, MU, st, h16, hbe, H, I, units, sorted_pos, tab, w, y, dk, zm); break;
+            default: launch_down<MOEHIP_PREC_BF16>(tok, MU, st, h16, hbe, H, I, units, sorted_pos, tab, w, y, dk, zm); break;
         }
     }
     if (xdtype == MOEHIP_DT_F16)
@@ -2186,16 +2427,16 @@ extern "C" int moehip_prefill_layer(int prec, const int64_t *tab, const void *x,
     int *xe = reinterpret_cast<int *>(wgg + G.xe);
     uint16_t *x16 = reinterpret_cast<uint16_t *>(wgg + G.x16);
     const uint16_t *xs = reinterpret_cast<const uint16_t *>(x);
-    const int prep = xdtype == MOEHIP_DT_BF16;
+    const int tok = gg_tokens(T * k, E), MU = gg_max_units(E, T * k, tok);
     const dim3 grid((T + 3) / 4);
     if (xdtype == MOEHIP_DT_F16)
         hipLaunchKernelGGL((k_route_post<MOEHIP_DT_F16>), grid, dim3(256), 0, st, logits, xs, T, H, E, k, renorm, idx, w,
-                           w32, cnt, bucket, xe, x16, prep);
+                           w32, cnt, bucket, xe, x16);
     else
         hipLaunchKernelGGL((k_route_post<MOEHIP_DT_BF16>), grid, dim3(256), 0, st, logits, xs, T, H, E, k, renorm, idx, w,
-                           w32, cnt, bucket, xe, x16, prep);
-    hipLaunchKernelGGL(k_route_place, dim3((T * k + 255) / 256), dim3(256), 0, st, cnt, bucket, T, k, E, counts, offsets,
-                       sorted, rank);
+                           w32, cnt, bucket, xe, x16);
+    hipLaunchKernelGGL(k_route_place, dim3((T * k + 255) / 256 + 1), dim3(256), 0, st, cnt, bucket, T, k, E, counts, offsets,
+                       sorted, rank, tok, MU, reinterpret_cast<int4 *>(wgg + G.units));
     // the combine (after every reader of the counters) leaves them zero
     return gg_run(1, &prec, tab, x, xdtype, T, H, I, k, E, gs, offsets, sorted, rank, w32, out, add, accumulate, wgg,
                   G.total, stream, 1, 0, nullptr, true, cnt, E, RP_STRIDE);
