@@ -73,6 +73,14 @@ int moehip_gemv_int4(const void *q, const void *s, const void *x, void *y, int O
 int moehip_dense_gemv_int8(const void *q, const void *s, const void *x, void *y, int O, int K, int gs, int dtype,
                            void *stream);
 /*
+ * The same for T tokens (a batched decode step's dense layers): y (T, O) = x W^T (+ bias (O)), x (T, K),
+ * bias (or NULL) and y in `dtype` (fp16 or bf16), on MFMA from the int8 weights (exact integer
+ * operands, fp32 sums and group scales, one rounding). K a multiple of 64, gs = 64; q and x 16-byte
+ * aligned. Replaces, for few tokens, the dequantise-then-F.linear of moelab/denseq.py:95-101.
+ */
+int moehip_dense_gemm_int8(const void *q, const void *s, const void *x, const void *bias, void *y, int T, int O, int K,
+                           int gs, int dtype, void *stream);
+/*
  * The multi-token path's weights: w (rows, K) in `dtype` = q * s for rows of the same int8 matrix,
  * the scale rounded to `dtype` first and the product rounded once (as moelab/quant.py:191-205
  * `dequantize(q, s, 8, dtype)` computes it). K a multiple of 16; q 16-byte aligned.

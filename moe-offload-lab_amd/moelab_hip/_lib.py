@@ -54,6 +54,7 @@ _SIGS = {
     "moehip_device_check": ([_i], _i),
     "moehip_gemv_int4": ([_vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp], _i),
     "moehip_dense_gemv_int8": ([_vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp], _i),
+    "moehip_dense_gemm_int8": ([_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp], _i),
     "moehip_dense_dequant_int8": ([_vp, _vp, _i, _i, _i, _i, _vp, _vp], _i),
     "moehip_grouped_up": ([_i, _vp, _vp, _vp, _i, _vp, _vp, _i, _i, _i, _i, _vp], _i),
     "moehip_grouped_down": ([_i, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp, _vp], _i),

@@ -24,6 +24,12 @@ __all__ = ["gemv_int8", "dequantize_rows", "quantize_int8", "QLinear", "quantiza
 # of the dequantisation kernel on every XCD) holding at most this many bytes of temporary weights.
 _ROWS_BUDGET_BYTES = 32 << 20
 
+# Tokens up to which the product runs straight from the int8 weights. The kernel reads them once per
+# 64 tokens; beyond this the dequantised weights and the library's product are faster (us, this kernel
+# / dequantised: 151936 x 2048 at 128 tokens 248 / 590, 256: 480 / 720, 512: 932 / 768; 50304 x 2048:
+# 94 / 213, 167 / 240, 313 / 255; 2048 x 4096: 26 / 40, 25 / 40, 45 / 41).
+FEW_TOKENS = 256
+
 
 def quantize_int8(w: torch.Tensor, group_size: int) -> tuple[torch.Tensor, torch.Tensor]:
     """(q (O, K) int8, s (O, K/gs) fp16) of a GPU matrix, symmetric per group (moelab/quant.py:129-170
@@ -65,8 +71,9 @@ class QLinear(nn.Module):
     dtype), keeping moelab's QLinear interface (denseq.py:69-109: `QLinear(q, s, group_size, bias,
     out_dtype)`, `from_linear`, the `q` / `s` buffers, `in_features` / `out_features`).
 
-    One token streams the int8 rows through moehip_dense_gemv_int8 (the bias added in place).
-    Several tokens compute the transposed product yT (out_features, tokens) one block of rows at
+    One token streams the int8 rows through moehip_dense_gemv_int8 (the bias added in place). Up to
+    FEW_TOKENS 16-bit tokens multiply straight from the int8 weights on MFMA (moehip_dense_gemm_int8).
+    More tokens compute the transposed product yT (out_features, tokens) one block of rows at
     a time: each block of W is dequantised into one reusable scratch matrix in the activation
     dtype (moehip_dense_dequant_int8, bit-identical to moelab's dequantize) and multiplied into
     its contiguous rows of yT by addmm with the bias folded in, so no partial results are
@@ -103,6 +110,23 @@ class QLinear(nn.Module):
             y.add_(self.bias.to(y.dtype))
         return y
 
+    def _few(self, x2: torch.Tensor) -> bool:
+        """Whether moehip_dense_gemm_int8 takes these tokens (an input that wants a gradient goes the
+        other way and is refused there, by the out= products)."""
+        return (x2.shape[0] <= FEW_TOKENS and x2.dtype in (torch.float16, torch.bfloat16) and self.group_size == 64
+                and self.in_features < 1 << 25 and x2.data_ptr() % 16 == 0 and self.q.data_ptr() % 16 == 0
+                and self.q.is_contiguous() and self.s.is_contiguous()
+                and not (x2.requires_grad and torch.is_grad_enabled()))
+
+    def _few_tokens(self, x2: torch.Tensor) -> torch.Tensor:
+        n = x2.shape[0]
+        y = torch.empty(n, self.out_features, dtype=x2.dtype, device=x2.device)
+        bias = None if self.bias is None else self.bias.to(x2.dtype)
+        _lib.call("moehip_dense_gemm_int8", self.q.data_ptr(), self.s.data_ptr(), x2.data_ptr(), _lib.ptr(bias),
+                  y.data_ptr(), n, self.out_features, self.in_features, 64, _lib.dt_code(x2.dtype),
+                  _lib.stream_of(x2.device))
+        return y
+
     def _tokens(self, x2: torch.Tensor) -> torch.Tensor:
         n = x2.shape[0]
         xt = x2.t()
@@ -137,7 +161,8 @@ class QLinear(nn.Module):
         if x2.shape[0] == 1 and self.kernel:
             y = self._one_token(x2.contiguous())
         else:
-            y = self._tokens(x2.contiguous())
+            x2 = x2.contiguous()
+            y = self._few_tokens(x2) if self._few(x2) else self._tokens(x2)
         return y.reshape(*lead, self.out_features)
 
     def extra_repr(self) -> str:
