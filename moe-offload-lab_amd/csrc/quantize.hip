@@ -47,6 +47,13 @@ __global__ __launch_bounds__(256) void k_quantize(const float *__restrict__ w, i
 // product, difference, quotient and fp16 conversion is rounded on its own: plain operators under
 // `fp contract(off)` (the __f*_rn helpers inline library code that may still be fused).
 //
+// Bound by VALU: 32 candidates per value, and the reference's correctly rounded division is half of
+// a candidate's ~19 operations. The search multiplies by the reciprocal instead (8 operations) and
+// divides only where that could change the integer (a quotient within its error of a half-integer that is no exact tie):
+// a 2048 x 2048 int4 matrix 72.6 -> 42.8 us, 2048 x 1024 40.7 -> 23.8 (18.1 M wave instructions a
+// launch on average, the VALU busy all the time). Dividing at exact ties too, which the lattice of
+// bf16 weights makes frequent, took 55.5; four candidates at a time 83 (one tie divides all four).
+//
 // 8 lanes per group (8 groups per wave): lane j holds the columns j, j + 8, ... below
 // gs - gs % 8, in the order of its running sum; every lane of the group also holds the last
 // gs % 8 columns. The group's lanes combine through DPP within their 8 lanes (xor 1, xor 2, the
@@ -83,10 +90,14 @@ __device__ __forceinline__ float tree8(float r) {
 // the factors: float(1.0 - 0.02 i) for i = 0..15 (the double expression rounded once)
 __constant__ const float kMseGrid[16] = {0x1p+0f, 0x1.f5c29p-1f, 0x1.eb851ep-1f, 0x1.e147aep-1f, 0x1.d70a3ep-1f, 0x1.ccccccp-1f, 0x1.c28f5cp-1f, 0x1.b851ecp-1f, 0x1.ae147ap-1f, 0x1.a3d70ap-1f, 0x1.99999ap-1f, 0x1.8f5c28p-1f, 0x1.851eb8p-1f, 0x1.7ae148p-1f, 0x1.70a3d8p-1f, 0x1.666666p-1f};
 
-__global__ __launch_bounds__(256) void k_quantize_mse(const float *__restrict__ w, int O, int I, int bits, int gs,
+// (GS = 64: the store's group size, straight-line code; 0: any, with the size's branches)
+template <int BITS, int GS>
+__global__ __launch_bounds__(256) void k_quantize_mse(const float *__restrict__ w, int O, int I, int gs_any,
                                                       uint8_t *__restrict__ q, uint16_t *__restrict__ s) {
     // no contraction: every product, difference and fp16 conversion rounds on its own
 #pragma clang fp contract(off)
+    constexpr int bits = BITS;
+    const int gs = GS ? GS : gs_any;
     const int j = threadIdx.x & 7;
     const int ng = I / gs;
     const long total = (long)O * ng;
@@ -124,32 +135,75 @@ __global__ __launch_bounds__(256) void k_quantize_mse(const float *__restrict__ 
     const float qmax = bits == 4 ? 7.f : 127.f, qmin = bits == 4 ? -8.f : -127.f;
     const uint16_t tiny = f32_to_f16_rne(1e-7f);
     const int nb = bits == 4 ? 2 : 1;
+    // x * rcp(s) is within 3 * 2^-23 of x / s relatively, the rounded quotient within 2^-24; in the
+    // range that is not clamped anyway |x / s| is below 16 (int4) or 256 (int8). Non-finite weights
+    // take the divided form (minimum, maximum and rint treat NaN in its own way there).
+    const float tie = 0.5f - (bits == 4 ? 16.f : 256.f) * 0x1p-21f;
+    float fin = 0.f;
+#pragma unroll
+    for (int m = 0; m < 8; ++m) fin = fin + v[m] * 0.f;
+#pragma unroll
+    for (int i = 0; i < 7; ++i) fin = fin + t[i] * 0.f;
+    const bool odd = fin != 0.f;  // NaN
+    const float grid = kMseGrid[threadIdx.x & 15];  // factor i in lane i
     uint16_t best_s = 0;
     float best_e = 0.f;
     for (int b = 0; b < nb; ++b) {
         const float bs = b == 0 ? a / qmax : sv / qmin;
+#pragma unroll 1
         for (int i = 0; i < 16; ++i) {
-            const float f = kMseGrid[i];
-            float bf = bs * f;
+            float bf = bs * lane_f(grid, i);
             asm volatile("" : "+v"(bf));  // the fp32 product itself (else fused into one fp16 rounding)
             uint16_t s16 = f32_to_f16_rne(bf);
             if ((s16 & 0x7fffu) == 0) s16 = tiny;
             const float sf = f16_to_f32(s16);
-            auto sq = [&](float x) {
-                const float qv = fminf(fmaxf(rintf(x / sf), qmin), qmax);
-                const float p = qv * sf;
-                const float d = p - x;
-                return d * d;
+            // the group's error with one squared term per value
+            auto total_of = [&](auto sq) {
+                float r = sq(v[0]);
+#pragma unroll
+                for (int m = 1; m < 8; ++m)
+                    if (m < n8) r = r + sq(v[m]);
+                float e = tree8(r);
+                if (n8 == 0) e = 0.f;
+#pragma unroll
+                for (int k = 0; k < 7; ++k)
+                    if (k < rem) e = e + sq(t[k]);
+                return e;
             };
-            float r = sq(v[0]);
+            // rint(x / s) from the reciprocal: the same integer unless the quotient is within the
+            // product's error of a half-integer (near: the largest distance of x * rcp(s) from its
+            // integer); k * s is exact (an integer of 8 bits times 11 bits), so fma(k, s, -x) is
+            // the rounded difference
+            const float ri = __builtin_amdgcn_rcpf(sf);
+            float near = 0.f;
+            float e = total_of([&](float x) {
+                const float tv = x * ri, kv = rintf(tv);
+                near = fmaxf(near, fabsf(tv - kv));
+                const float d = fmaf(__builtin_amdgcn_fmed3f(kv, qmin, qmax), sf, -x);
+                return d * d;
+            });
+            if (__builtin_amdgcn_ballot_w64(near > tie || odd) != 0ull) {
+                // an exact tie (|x - k s| = s / 2: frequent with bf16 weights) has the same squared
+                // difference for either integer; only an inexact one needs the division
+                bool inexact = odd;
+                auto look = [&](float x) {
+                    const float tv = x * ri, kv = rintf(tv);
+                    inexact |= fabsf(tv - kv) > tie && 2.f * fabsf(fmaf(kv, sf, -x)) != fabsf(sf);
+                };
 #pragma unroll
-            for (int m = 1; m < 8; ++m)
-                if (m < n8) r = r + sq(v[m]);
-            float e = tree8(r);
-            if (n8 == 0) e = 0.f;
+                for (int m = 0; m < 8; ++m)
+                    if (m < n8) look(v[m]);
 #pragma unroll
-            for (int k = 0; k < 7; ++k)
-                if (k < rem) e = e + sq(t[k]);
+                for (int k = 0; k < 7; ++k)
+                    if (k < rem) look(t[k]);
+                if (__builtin_amdgcn_ballot_w64(inexact) != 0ull)
+                    e = total_of([&](float x) {
+                        const float qv = fminf(fmaxf(rintf(x / sf), qmin), qmax);
+                        const float p = qv * sf;
+                        const float d = p - x;
+                        return d * d;
+                    });
+            }
             if ((b == 0 && i == 0) || e < best_e) {
                 best_e = e;
                 best_s = s16;
@@ -256,7 +310,13 @@ extern "C" int moehip_quantize_mse(const float *w, int O, int I, int bits, int g
     MOEHIP_REQUIRE(O > 0 && I > 0 && gs > 0 && gs <= 64 && gs % 2 == 0 && I % gs == 0,
                    "quantize_mse: bad sizes O=%d I=%d gs=%d", O, I, gs);
     const long groups = (long)O * (I / gs);
-    hipLaunchKernelGGL(k_quantize_mse, dim3((unsigned)((groups + 31) / 32)), dim3(256), 0, as_stream(stream), w, O, I,
-                       bits, gs, reinterpret_cast<uint8_t *>(q), reinterpret_cast<uint16_t *>(s));
+    const dim3 grid((unsigned)((groups + 31) / 32));
+    uint8_t *qb = reinterpret_cast<uint8_t *>(q);
+    uint16_t *sh = reinterpret_cast<uint16_t *>(s);
+    hipStream_t st = as_stream(stream);
+    if (bits == 4 && gs == 64) hipLaunchKernelGGL((k_quantize_mse<4, 64>), grid, dim3(256), 0, st, w, O, I, gs, qb, sh);
+    else if (bits == 4) hipLaunchKernelGGL((k_quantize_mse<4, 0>), grid, dim3(256), 0, st, w, O, I, gs, qb, sh);
+    else if (gs == 64) hipLaunchKernelGGL((k_quantize_mse<8, 64>), grid, dim3(256), 0, st, w, O, I, gs, qb, sh);
+    else hipLaunchKernelGGL((k_quantize_mse<8, 0>), grid, dim3(256), 0, st, w, O, I, gs, qb, sh);
     return check_launch("quantize_mse");
 }
