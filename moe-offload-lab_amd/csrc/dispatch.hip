@@ -82,11 +82,16 @@ __device__ __forceinline__ void dispatch_wg(const int64_t *__restrict__ idx, con
     }
     __syncthreads();
     // per expert: column prefix over the waves (wave starts relative to the expert's offset)
+    // (the column is read at once: a read behind each write would be NW round trips of the LDS)
     int tot = 0;  // E <= 1024: thread e owns expert e
+    int col[DP_WAVES];
     if (tid < E) {
-        for (int w = 0; w < NW; ++w) {
-            const int c = s_cnt[w * E + tid];
-            s_cnt[w * E + tid] = tot;
+#pragma unroll
+        for (int w = 0; w < DP_WAVES; ++w) col[w] = s_cnt[min(w, NW - 1) * E + tid];
+#pragma unroll
+        for (int w = 0; w < DP_WAVES; ++w) {
+            const int c = w < NW ? col[w] : 0;
+            col[w] = tot;
             tot += c;
         }
         counts[tid] = tot;
@@ -104,7 +109,9 @@ __device__ __forceinline__ void dispatch_wg(const int64_t *__restrict__ idx, con
     const int excl = wbase + incl - tot;
     if (tid < E) {
         offsets[tid] = excl;
-        for (int w = 0; w < NW; ++w) s_cnt[w * E + tid] += excl;
+#pragma unroll
+        for (int w = 0; w < DP_WAVES; ++w)
+            if (w < NW) s_cnt[w * E + tid] = col[w] + excl;
         if (tid == E - 1) offsets[E] = excl + tot;
     }
     int total = 0;
@@ -375,6 +382,12 @@ __device__ __forceinline__ void write_items_1k(int ch, int n, int EA, int np, in
 // levels per (token, slot) (one wave per token, slot_level), the dispatch of the kept pairs over
 // the E + has_shared experts, and the vote / copy / tables per expert (vote_expert); the same
 // results as moehip_batch_levels + moehip_dispatch + moehip_batch_vote.
+// LEVELS: the levels are made here, one wave per token after another; else moehip_batch_levels has
+// made them over the whole chip (more than DP_LEVEL_TOKENS tokens) and this launch only tallies them,
+// a pair per thread. Alone, us: 32 tokens x 11 slots 7.0 here; 100 x 11 13.3 -> 13.0; 512 x 8 24.7
+// (weight threshold) / 62.1 (HOBBIT's ranking) -> 14.0 / 14.7.
+constexpr int DP_LEVEL_TOKENS = 64;
+template <bool LEVELS>
 __global__ __launch_bounds__(1024) void k_batch_decide(const float *__restrict__ w, const int64_t *__restrict__ idx,
                                                        int T, int k, int ks, moehip_policy pol,
                                                        int32_t *__restrict__ levels, uint8_t *__restrict__ skip, int E,
@@ -397,8 +410,33 @@ __global__ __launch_bounds__(1024) void k_batch_decide(const float *__restrict__
     vote_recs(vr, tid, E, EA, rtab, srec, P, offs, planned);
     tally_clear(s_vt, EA);
     __syncthreads();
-    for (int t = wave; t < T; t += DP_WAVES)
-        token_levels(t, k, ks, EA, w, idx, pol, levels, skip, s_w[wave], s_sorted[wave], &s_total[wave], s_vt, pe);
+    if constexpr (LEVELS) {
+        for (int t = wave; t < T; t += DP_WAVES)
+            token_levels(t, k, ks, EA, w, idx, pol, levels, skip, s_w[wave], s_sorted[wave], &s_total[wave], s_vt, pe);
+    } else {
+        constexpr int U = 4;  // pairs per thread whose loads are in flight together
+        const int NP = T * ks;
+        for (int q0 = tid; q0 < NP; q0 += U * 1024) {
+            int64_t e[U];
+            int lvl[U];
+            bool sk[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int q = min(q0 + u * 1024, NP - 1);
+                e[u] = idx[q];
+                lvl[u] = levels[q];
+                sk[u] = skip[q] != 0;
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int q = q0 + u * 1024;
+                if (q >= NP) break;
+                const bool kept = !sk[u] && e[u] >= 0 && e[u] < EA;
+                if (kept) tally_add(s_vt, (int)e[u], lvl[u]);
+                if (pe != nullptr) pe[q] = kept ? (int16_t)e[u] : (int16_t)-1;
+            }
+        }
+    }
     __syncthreads();
     if (T * ks <= 64 && EA <= 64) {
         if (wave == 0) dispatch_wave64(idx, skip, T * ks, EA, ebits, counts, offsets, sorted_pos, rank, s_cnt, pe);
@@ -542,11 +580,20 @@ extern "C" int moehip_batch_decide(const float *w32, const int64_t *idx, int T, 
     int ebits = 0;
     while ((1 << ebits) < EA) ++ebits;
     const size_t lds = (size_t)DP_WAVES * EA * sizeof(int);
-    MOEHIP_REQUIRE(enable_big_lds(reinterpret_cast<const void *>(&k_batch_decide), lds),
+    MOEHIP_REQUIRE(enable_big_lds(reinterpret_cast<const void *>(&k_batch_decide<true>), lds) &&
+                       enable_big_lds(reinterpret_cast<const void *>(&k_batch_decide<false>), lds),
                    "batch_decide: cannot enable %zu bytes of LDS", lds);
-    hipLaunchKernelGGL(k_batch_decide, dim3(1), dim3(1024), lds, as_stream(stream), w32, idx, T, k, ks, *pol, levels,
-                       skip, E, has_shared ? 1 : 0, ebits, counts, offsets, sorted_pos, rank, hi_vote, lv2p[0], lv2p[1],
-                       lv2p[2], rtab, sr, P, offs, planned, tabs, info, miss, items);
+    if (T <= DP_LEVEL_TOKENS) {
+        hipLaunchKernelGGL(k_batch_decide<true>, dim3(1), dim3(1024), lds, as_stream(stream), w32, idx, T, k, ks, *pol, levels,
+                           skip, E, has_shared ? 1 : 0, ebits, counts, offsets, sorted_pos, rank, hi_vote, lv2p[0], lv2p[1],
+                           lv2p[2], rtab, sr, P, offs, planned, tabs, info, miss, items);
+    } else {
+        const int rc = moehip_batch_levels(w32, T, k, ks, pol, levels, skip, stream);
+        if (rc != MOEHIP_OK) return rc;
+        hipLaunchKernelGGL(k_batch_decide<false>, dim3(1), dim3(1024), lds, as_stream(stream), w32, idx, T, k, ks, *pol, levels,
+                           skip, E, has_shared ? 1 : 0, ebits, counts, offsets, sorted_pos, rank, hi_vote, lv2p[0], lv2p[1],
+                           lv2p[2], rtab, sr, P, offs, planned, tabs, info, miss, items);
+    }
     return check_launch("batch_decide");
 }
 
