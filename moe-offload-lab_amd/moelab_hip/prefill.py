@@ -116,6 +116,31 @@ class GroupedTokens:
         return out
 
 
+# Batched GEMVs or MFMA tiles. The GEMVs run each (token, expert) pair on its own and cost about
+# c + pairs x record / 9.3 TB/s (an expert's further tokens re-read its record from the caches); the
+# tiles read an expert's record once however many tokens it has, c' + experts x record / 4.6 TB/s with
+# c' - c of 10 us and more (the activations' preparation, fewer workgroups). So the GEMVs pay up to
+# RATIO x (distinct experts) + EXTRA / record pairs, by the kind of the least precise record (fp8 rows
+# cost the GEMVs more, 16-bit rows the tiles). us per layer, GEMVs / tiles, on either side of the line:
+#   int4  64 experts top-8 (d_ff 1024): 16 tokens 85 / 83, 24: 105 / 86, 64: 218 / 89;  128 experts top-8
+#         (768): 32: 118 / 111;  512 top-10 + shared (512): 64: 184 / 200, 96: 250 / 232
+#   int8  64 experts: 16: 119 / 123, 20: 136 / 125;  512: 64: 298 / 313
+#   fp8   64 experts: 12: 110 / 108, 16: 130 / 113;  128: 16: 116 / 135, 32: 188 / 151;  512: 48: 246 / 247,
+#         64: 308 / 267;  16 top-4 (512): 16: 52 / 59, 32: 76 / 61
+#   fp16  64 experts: 20: 191 / 195, 24: 211 / 197;  16 top-4 (1024): 16: 87 / 101, 32: 121 / 99
+#   fp16 + int4 (weight rule)  64 experts: 16: 129 / 150, 24: 175 / 110;  128: 32: 218 / 284, 48: 291 / 261
+GEMV_RATIO_EXTRA = {"int4": (2.0, 93e6), "int8": (2.0, 150e6), "fp8": (1.7, 150e6), "fp16": (2.3, 400e6),
+                    "bf16": (2.3, 400e6)}
+
+
+def gemv_pays(T: int, k: int, E: int, shared: bool, kind: str, record_bytes: int) -> bool:
+    """Whether T tokens' top-k pairs over E experts (and a shared one) are fewer than the line above, with
+    the distinct experts expected of uniform routing."""
+    ratio, extra = GEMV_RATIO_EXTRA[kind]
+    distinct = E * (1.0 - (1.0 - k / E) ** T) + (1 if shared else 0)
+    return T * (k + (1 if shared else 0)) <= ratio * distinct + extra / record_bytes
+
+
 class GroupedLayer:
     """T > 1 tokens (batched decode of a few tokens, prefill chunks) through the MoE layers of a
     `ResidentStore` on the GPU, any record precision and one precision per expert.
@@ -133,9 +158,9 @@ class GroupedLayer:
          router runs here on up to route_fused_tokens 16-bit tokens, the top-k, 2, 3-5 and the
          GEMVs' work list in one launch after the logits (moehip_router_logits +
          moehip_batch_route_decide)
-      6. expert products per precision + ordered combine: batched dequant GEMVs for up to
-         `gemv_tokens` tokens (moehip_grouped_gemv_multi), MFMA tiles beyond
-         (moehip_grouped_gemm_multi)
+      6. expert products per precision + ordered combine: batched dequant GEMVs
+         (moehip_grouped_gemv_multi) for up to `gemv_tokens` tokens while they pay (`gemv_pays`),
+         MFMA tiles beyond (moehip_grouped_gemm_multi)
     `shared`: per layer None or {"gate": (H,) tensor in dtype, "rec": {precision: record blob}}
     (the same form as MoEDecoder's). `info[layer]` (E + 1) holds the precision index each expert
     ran at (-1 missing, -2 no pairs); `miss` counts pairs of experts with no usable copy."""
@@ -246,7 +271,7 @@ class GroupedLayer:
             pidx, pw, ks, EA = self.idx_ext, self.w_ext, k + 1, self.E + 1
         else:
             pidx, pw, ks, EA = idx, w32, k, self.E
-        gemv = T <= self.gemv_tokens
+        gemv = self._gemv(T, srec is not None)
         items = None
         if self.fused_decide:
             items = self.items.data_ptr() if gemv else None
@@ -270,6 +295,10 @@ class GroupedLayer:
             _lib.call("moehip_grouped_gemm_multi", *args, stream)
         return out
 
+    def _gemv(self, T: int, shared: bool) -> bool:
+        low = self.store.layouts[self.store.precisions[-1]]
+        return T <= self.gemv_tokens and gemv_pays(T, self.k, self.E, shared, low["precision"], low["record_bytes"])
+
     def _decide(self, layer, pw, pidx, T, ks, srec, items, stream):
         _lib.call("moehip_batch_decide", pw.data_ptr(), pidx.data_ptr(), T, self.k, ks,
                   ctypes.byref(self._pols[layer]), self.levels.data_ptr(), self.skip.data_ptr(), self.E,
@@ -291,7 +320,7 @@ class GroupedLayer:
         _lib.call("moehip_router_logits", x.data_ptr(), Wr.data_ptr(), T, self.H, self.E, dt, self.logits.data_ptr(),
                   stream)
         g = self.shared[layer]["gate"] if shared else None
-        gemv = T <= self.gemv_tokens
+        gemv = self._gemv(T, srec is not None)
         if T > self.route_fused_tokens:
             _lib.call("moehip_route_tokens", self.logits.data_ptr(), dt, T, self.E, k, 1 if self.renorm else 0,
                       x.data_ptr(), _lib.ptr(g), self.H, self.idx.data_ptr(), self.w.data_ptr(), self.w32.data_ptr(),
