@@ -225,6 +225,15 @@ int moehip_quantize(const float *w, int O, int I, int bits, int gs, void *q, voi
 int moehip_quantize_mse(const float *w, int O, int I, int bits, int gs, void *q, void *s, void *stream);
 
 /*
+ * The three quantisers on weights as a checkpoint holds them: w (O, I) in wdtype (fp16, bf16 or
+ * fp32, widened exactly), prec = MOEHIP_PREC_INT4 / INT8 (absmax, or mse != 0: moehip_quantize_mse's
+ * search) or FP8 (moehip_quantize_fp8_block; gs and mse ignored); q and s as those entries write
+ * them. Replaces the float32 copy of moelab/store.py:122-150 in front of the quantiser.
+ */
+int moehip_quantize_weights(const void *w, int wdtype, int O, int I, int prec, int gs, int mse, void *q, void *s,
+                            void *stream);
+
+/*
  * GPTQ column sweep of one block (moelab/quant.py:172-186, inside gptq_quantize, quant.py:130-188):
  * rows 0..O-1 of W (float32, row stride ldw), columns i1 .. i1 + nb - 1 (nb <= 128, i1 and nb
  * multiples of gs = 32 or 64), against the block of Hinv (the upper Cholesky factor of H^-1, row

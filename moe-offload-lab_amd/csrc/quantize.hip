@@ -7,7 +7,10 @@
 
 namespace moehip {
 
-__global__ __launch_bounds__(256) void k_quantize(const float *__restrict__ w, int O, int I, int bits, int gs,
+// The weights come in fp32, fp16 or bf16 (WDT): read as a checkpoint holds them, widened exactly in
+// registers. (Float32 copies and a cleared record first were 17 us of the 78 per OLMoE expert.)
+template <int WDT>
+__global__ __launch_bounds__(256) void k_quantize(const void *__restrict__ w, int O, int I, int bits, int gs,
                                                   uint8_t *__restrict__ q, uint16_t *__restrict__ s) {
     const int lane = threadIdx.x & 63;
     const int ng = I / gs;
@@ -15,7 +18,7 @@ __global__ __launch_bounds__(256) void k_quantize(const float *__restrict__ w, i
     if (gid >= (long)O * ng) return;
     const int row = (int)(gid / ng), g = (int)(gid % ng);
     const bool act = lane < gs;
-    const float v = act ? w[(size_t)row * I + (size_t)g * gs + lane] : 0.f;
+    const float v = act ? ld_act<WDT>(w, (size_t)row * I + (size_t)g * gs + lane) : 0.f;
     const float amax = wave_max(fabsf(v));
     const float qmax = bits == 4 ? 7.f : 127.f;
     const float qmin = bits == 4 ? -8.f : -127.f;
@@ -91,8 +94,8 @@ __device__ __forceinline__ float tree8(float r) {
 __constant__ const float kMseGrid[16] = {0x1p+0f, 0x1.f5c29p-1f, 0x1.eb851ep-1f, 0x1.e147aep-1f, 0x1.d70a3ep-1f, 0x1.ccccccp-1f, 0x1.c28f5cp-1f, 0x1.b851ecp-1f, 0x1.ae147ap-1f, 0x1.a3d70ap-1f, 0x1.99999ap-1f, 0x1.8f5c28p-1f, 0x1.851eb8p-1f, 0x1.7ae148p-1f, 0x1.70a3d8p-1f, 0x1.666666p-1f};
 
 // (GS = 64: the store's group size, straight-line code; 0: any, with the size's branches)
-template <int BITS, int GS>
-__global__ __launch_bounds__(256) void k_quantize_mse(const float *__restrict__ w, int O, int I, int gs_any,
+template <int BITS, int GS, int WDT>
+__global__ __launch_bounds__(256) void k_quantize_mse(const void *__restrict__ w, int O, int I, int gs_any,
                                                       uint8_t *__restrict__ q, uint16_t *__restrict__ s) {
     // no contraction: every product, difference and fp16 conversion rounds on its own
 #pragma clang fp contract(off)
@@ -105,13 +108,13 @@ __global__ __launch_bounds__(256) void k_quantize_mse(const float *__restrict__ 
     const bool live = gid < total;
     const long gg = live ? gid : 0;
     const int row = (int)(gg / ng), g = (int)(gg % ng);
-    const float *src = w + (size_t)row * I + (size_t)g * gs;
+    const size_t src = (size_t)row * I + (size_t)g * gs;
     const int n8 = gs >> 3, rem = gs & 7, base = gs - rem;
     float v[8], t[7];
 #pragma unroll
-    for (int m = 0; m < 8; ++m) v[m] = m < n8 ? src[j + 8 * m] : 0.f;
+    for (int m = 0; m < 8; ++m) v[m] = m < n8 ? ld_act<WDT>(w, src + j + 8 * m) : 0.f;
 #pragma unroll
-    for (int i = 0; i < 7; ++i) t[i] = i < rem ? src[base + i] : 0.f;
+    for (int i = 0; i < 7; ++i) t[i] = i < rem ? ld_act<WDT>(w, src + base + i) : 0.f;
     // the largest magnitude and the signed value at its first index
     float a = -1.f, sv = 0.f;
     int ix = 1 << 30;
@@ -258,7 +261,8 @@ __device__ __forceinline__ uint32_t f32_to_e4m3fn(float x) {
 
 // Checkpoint-style FP8 block quantisation: one workgroup per 128 x 128 block,
 // scale = amax / 448 (1 for an all-zero block), code = e4m3fn(w / scale).
-__global__ __launch_bounds__(256) void k_quantize_fp8_block(const float *__restrict__ w, int O, int I,
+template <int WDT>
+__global__ __launch_bounds__(256) void k_quantize_fp8_block(const void *__restrict__ w, int O, int I,
                                                             uint8_t *__restrict__ q, float *__restrict__ s) {
     __shared__ float s_max[4];
     const int bo = blockIdx.y, bi = blockIdx.x;
@@ -267,7 +271,7 @@ __global__ __launch_bounds__(256) void k_quantize_fp8_block(const float *__restr
     float m = 0.f;
     for (int t = tid; t < 128 * 128; t += 256) {
         const int r = bo * 128 + (t >> 7), c = bi * 128 + (t & 127);
-        if (r < O && c < I) m = fmaxf(m, fabsf(w[(size_t)r * I + c]));
+        if (r < O && c < I) m = fmaxf(m, fabsf(ld_act<WDT>(w, (size_t)r * I + c)));
     }
     m = wave_max(m);
     if ((tid & 63) == 0) s_max[tid >> 6] = m;
@@ -277,7 +281,7 @@ __global__ __launch_bounds__(256) void k_quantize_fp8_block(const float *__restr
     if (tid == 0) s[(size_t)bo * sc + bi] = scale;
     for (int t = tid; t < 128 * 128; t += 256) {
         const int r = bo * 128 + (t >> 7), c = bi * 128 + (t & 127);
-        if (r < O && c < I) q[(size_t)r * I + c] = (uint8_t)f32_to_e4m3fn(w[(size_t)r * I + c] / scale);
+        if (r < O && c < I) q[(size_t)r * I + c] = (uint8_t)f32_to_e4m3fn(ld_act<WDT>(w, (size_t)r * I + c) / scale);
     }
 }
 
@@ -285,38 +289,52 @@ __global__ __launch_bounds__(256) void k_quantize_fp8_block(const float *__restr
 
 using namespace moehip;
 
-extern "C" int moehip_quantize_fp8_block(const float *w, int O, int I, void *q, float *s, void *stream) {
-    MOEHIP_REQUIRE(w && q && s, "quantize_fp8_block: null pointer");
-    MOEHIP_REQUIRE(O > 0 && I > 0, "quantize_fp8_block: bad sizes O=%d I=%d", O, I);
-    hipLaunchKernelGGL(k_quantize_fp8_block, dim3((I + 127) / 128, (O + 127) / 128), dim3(256), 0, as_stream(stream), w,
-                       O, I, reinterpret_cast<uint8_t *>(q), s);
-    return check_launch("quantize_fp8_block");
+template <int WDT>
+static void launch_quantize(const void *w, int O, int I, int prec, int gs, int mse, void *q, void *s, hipStream_t st) {
+    if (prec == MOEHIP_PREC_FP8) {
+        hipLaunchKernelGGL((k_quantize_fp8_block<WDT>), dim3((I + 127) / 128, (O + 127) / 128), dim3(256), 0, st, w, O, I,
+                           reinterpret_cast<uint8_t *>(q), reinterpret_cast<float *>(s));
+        return;
+    }
+    const long groups = (long)O * (I / gs);
+    uint8_t *qb = reinterpret_cast<uint8_t *>(q);
+    uint16_t *sh = reinterpret_cast<uint16_t *>(s);
+    const int bits = prec == MOEHIP_PREC_INT4 ? 4 : 8;
+    if (!mse) {
+        hipLaunchKernelGGL((k_quantize<WDT>), dim3((unsigned)((groups + 3) / 4)), dim3(256), 0, st, w, O, I, bits, gs, qb, sh);
+        return;
+    }
+    const dim3 grid((unsigned)((groups + 31) / 32));
+    if (bits == 4 && gs == 64) hipLaunchKernelGGL((k_quantize_mse<4, 64, WDT>), grid, dim3(256), 0, st, w, O, I, gs, qb, sh);
+    else if (bits == 4) hipLaunchKernelGGL((k_quantize_mse<4, 0, WDT>), grid, dim3(256), 0, st, w, O, I, gs, qb, sh);
+    else if (gs == 64) hipLaunchKernelGGL((k_quantize_mse<8, 64, WDT>), grid, dim3(256), 0, st, w, O, I, gs, qb, sh);
+    else hipLaunchKernelGGL((k_quantize_mse<8, 0, WDT>), grid, dim3(256), 0, st, w, O, I, gs, qb, sh);
 }
 
-extern "C" int moehip_quantize(const float *w, int O, int I, int bits, int gs, void *q, void *s, void *stream) {
+extern "C" int moehip_quantize_weights(const void *w, int wdtype, int O, int I, int prec, int gs, int mse, void *q, void *s,
+                                       void *stream) {
     MOEHIP_REQUIRE(w && q && s, "quantize: null pointer");
-    MOEHIP_REQUIRE(bits == 4 || bits == 8, "quantize: bits must be 4 or 8, got %d", bits);
-    MOEHIP_REQUIRE(O > 0 && I > 0 && gs > 0 && gs <= 64 && gs % 2 == 0 && I % gs == 0,
+    MOEHIP_REQUIRE(wdtype >= MOEHIP_DT_F16 && wdtype <= MOEHIP_DT_F32, "quantize: weight dtype %d", wdtype);
+    MOEHIP_REQUIRE(prec == MOEHIP_PREC_INT4 || prec == MOEHIP_PREC_INT8 || prec == MOEHIP_PREC_FP8, "quantize: record precision %d", prec);
+    MOEHIP_REQUIRE(O > 0 && I > 0 && (prec == MOEHIP_PREC_FP8 || (gs > 0 && gs <= 64 && gs % 2 == 0 && I % gs == 0)),
                    "quantize: bad sizes O=%d I=%d gs=%d", O, I, gs);
-    const long groups = (long)O * (I / gs);
-    hipLaunchKernelGGL(k_quantize, dim3((unsigned)((groups + 3) / 4)), dim3(256), 0, as_stream(stream), w, O, I, bits, gs,
-                       reinterpret_cast<uint8_t *>(q), reinterpret_cast<uint16_t *>(s));
+    hipStream_t st = as_stream(stream);
+    if (wdtype == MOEHIP_DT_F16) launch_quantize<MOEHIP_DT_F16>(w, O, I, prec, gs, mse, q, s, st);
+    else if (wdtype == MOEHIP_DT_BF16) launch_quantize<MOEHIP_DT_BF16>(w, O, I, prec, gs, mse, q, s, st);
+    else launch_quantize<MOEHIP_DT_F32>(w, O, I, prec, gs, mse, q, s, st);
     return check_launch("quantize");
 }
 
+extern "C" int moehip_quantize_fp8_block(const float *w, int O, int I, void *q, float *s, void *stream) {
+    return moehip_quantize_weights(w, MOEHIP_DT_F32, O, I, MOEHIP_PREC_FP8, 0, 0, q, s, stream);
+}
+
+extern "C" int moehip_quantize(const float *w, int O, int I, int bits, int gs, void *q, void *s, void *stream) {
+    MOEHIP_REQUIRE(bits == 4 || bits == 8, "quantize: bits must be 4 or 8, got %d", bits);
+    return moehip_quantize_weights(w, MOEHIP_DT_F32, O, I, bits == 4 ? MOEHIP_PREC_INT4 : MOEHIP_PREC_INT8, gs, 0, q, s, stream);
+}
+
 extern "C" int moehip_quantize_mse(const float *w, int O, int I, int bits, int gs, void *q, void *s, void *stream) {
-    MOEHIP_REQUIRE(w && q && s, "quantize_mse: null pointer");
     MOEHIP_REQUIRE(bits == 4 || bits == 8, "quantize_mse: bits must be 4 or 8, got %d", bits);
-    MOEHIP_REQUIRE(O > 0 && I > 0 && gs > 0 && gs <= 64 && gs % 2 == 0 && I % gs == 0,
-                   "quantize_mse: bad sizes O=%d I=%d gs=%d", O, I, gs);
-    const long groups = (long)O * (I / gs);
-    const dim3 grid((unsigned)((groups + 31) / 32));
-    uint8_t *qb = reinterpret_cast<uint8_t *>(q);
-    uint16_t *sh = reinterpret_cast<uint16_t *>(s);
-    hipStream_t st = as_stream(stream);
-    if (bits == 4 && gs == 64) hipLaunchKernelGGL((k_quantize_mse<4, 64>), grid, dim3(256), 0, st, w, O, I, gs, qb, sh);
-    else if (bits == 4) hipLaunchKernelGGL((k_quantize_mse<4, 0>), grid, dim3(256), 0, st, w, O, I, gs, qb, sh);
-    else if (gs == 64) hipLaunchKernelGGL((k_quantize_mse<8, 64>), grid, dim3(256), 0, st, w, O, I, gs, qb, sh);
-    else hipLaunchKernelGGL((k_quantize_mse<8, 0>), grid, dim3(256), 0, st, w, O, I, gs, qb, sh);
-    return check_launch("quantize_mse");
+    return moehip_quantize_weights(w, MOEHIP_DT_F32, O, I, bits == 4 ? MOEHIP_PREC_INT4 : MOEHIP_PREC_INT8, gs, 1, q, s, stream);
 }

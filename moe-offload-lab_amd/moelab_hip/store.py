@@ -139,7 +139,11 @@ def encode_record_(layout: dict, blob: torch.Tensor, gate_up: torch.Tensor, down
     spec = PRECISIONS[prec]
     if blob.numel() != layout["record_bytes"] or blob.dtype != torch.uint8:
         raise ValueError("blob must be a uint8 tensor of record_bytes")
-    blob.zero_()
+    gaps = _padding(layout)
+    if len(gaps) == 1:  # the fields below cover the rest
+        blob[gaps[0][0]:gaps[0][1]].zero_()
+    elif gaps:
+        blob.zero_()
     v = views(layout, blob)
     mats = {"gate_up": gate_up, "down": down}
     if spec["kind"] == "float":
@@ -149,25 +153,29 @@ def encode_record_(layout: dict, blob: torch.Tensor, gate_up: torch.Tensor, down
     if blob.device.type != "cuda":
         raise RuntimeError("encode_record_ quantises on the GPU; blob must be a device tensor")
     _lib.check_device(blob.device)
-    if spec["kind"] == "fp8":
-        for name, w in mats.items():
-            wf = w.float().contiguous()
-            O, I = wf.shape
-            _lib.call("moehip_quantize_fp8_block", wf.data_ptr(), O, I, v[f"{name}.q"].data_ptr(),
-                      v[f"{name}.s"].data_ptr(), _lib.stream_of(blob.device))
-        return blob
-    bits = spec["bits"]
     method = layout.get("scale") or "absmax"
-    if method not in ("absmax", "mse"):
+    if spec["kind"] == "int" and method not in ("absmax", "mse"):
         raise ValueError(f"unknown scale method {method!r} (absmax, mse)")
-    entry = "moehip_quantize_mse" if method == "mse" else "moehip_quantize"
     for name, w in mats.items():
-        wf = w.float().contiguous()
+        # 16-bit weights are widened by the quantiser itself
+        wf = (w if w.dtype in _lib.DT_CODES else w.float()).contiguous()
         O, I = wf.shape
-        gs = layout["group_sizes"][name]
-        _lib.call(entry, wf.data_ptr(), O, I, bits, gs, v[f"{name}.q"].data_ptr(),
-                  v[f"{name}.s"].data_ptr(), _lib.stream_of(blob.device))
+        _lib.call("moehip_quantize_weights", wf.data_ptr(), _lib.dt_code(wf.dtype), O, I, _lib.prec_code(prec),
+                  layout["group_sizes"].get(name, 0), 1 if spec["kind"] == "int" and method == "mse" else 0,
+                  v[f"{name}.q"].data_ptr(), v[f"{name}.s"].data_ptr(), _lib.stream_of(blob.device))
     return blob
+
+
+def _padding(layout: dict) -> list[tuple[int, int]]:
+    """Byte ranges of a record that no field covers."""
+    gaps, end = [], 0
+    for _, shape, dtype, off in layout["fields"]:
+        if off > end:
+            gaps.append((end, off))
+        end = off + ELEM_SIZE[dtype] * math.prod(shape)
+    if layout["record_bytes"] > end:
+        gaps.append((end, layout["record_bytes"]))
+    return gaps
 
 
 def unpacked_layout(layout: dict) -> dict | None:

@@ -36,3 +36,23 @@ def test_mse_at_half_integers(dev, bits, gs):
     q_ref, s_ref = O.quantize(w, bits, gs, "mse")
     assert np.array_equal(s.cpu().numpy().view(np.uint16), np.asarray(s_ref).view(np.uint16))
     assert np.array_equal(q.cpu().numpy().view(np.uint8), np.asarray(q_ref).view(np.uint8))
+
+
+@pytest.mark.parametrize("prec,scale", [("int4", "mse"), ("int4", "absmax"), ("int8", "mse"), ("int8", "absmax"),
+                                        ("fp8", None), ("fp16", None)])
+@pytest.mark.parametrize("H,I", [(256, 128), (192, 100), (130, 66)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_encode_record_from_16_bit_weights(dev, prec, scale, H, I, dtype):
+    """A record encoded from 16-bit weights (widened in the quantiser) into a used buffer: the bytes of
+    the same record encoded from their float32 copies into a fresh one, its padding zero."""
+    from moelab_hip.store import encode_record_, record_layout
+
+    lay = record_layout(prec, H, I, 64, scale=scale)
+    g = torch.Generator().manual_seed(H + I)
+    gu = (torch.randn(2 * I, H, generator=g) * 0.02).to(dtype).to(dev)
+    dn = (torch.randn(H, I, generator=g) * 0.02).to(dtype).to(dev)
+    ref = encode_record_(lay, torch.zeros(lay["record_bytes"], dtype=torch.uint8, device=dev), gu.float(), dn.float())
+    got = encode_record_(lay, torch.full((lay["record_bytes"],), 0xA5, dtype=torch.uint8, device=dev), gu, dn)
+    # a view with other strides: made contiguous first
+    got2 = encode_record_(lay, torch.full_like(got, 0x5A), gu.t().contiguous().t(), dn)
+    assert torch.equal(ref, got) and torch.equal(ref, got2)
