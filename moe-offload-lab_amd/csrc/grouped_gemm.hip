@@ -559,6 +559,33 @@ __device__ __forceinline__ float half_max(float f) {
     return __uint_as_float(v);
 }
 
+// A launch runs one record table (PB < 0) or both of a two-precision store, whose second table is E
+// rows further (the later row counts, as with a launch for each). A launch per precision left the chip
+// to the other kind's few experts, or cost ~5 us with none: 16-bit + int4 layer, 128 experts of d_model
+// 2048 and d_ff 768, 64 tokens, 19 experts at 16 bits: 253 -> 196 us; 64 experts of d_ff 1024, 1024
+// tokens, all at int4: 247 -> 240. `tile` gets the record kind as a constant and the fields f, f + 1
+// of the row; false: no row.
+constexpr int gg_ck(int pa, int pb) {
+    auto ck = [](int p) { return p == MOEHIP_PREC_INT4 ? 128 : (p == MOEHIP_PREC_INT8 || p == MOEHIP_PREC_FP8) ? 64 : 32; };
+    return pb < 0 || ck(pa) > ck(pb) ? ck(pa) : ck(pb);
+}
+template <int PA, int PB, class F>
+__device__ __forceinline__ bool gg_tables(const int64_t *tab, int E, int e, int f, F &&tile) {
+    const int64_t *ra = tab + 4 * (size_t)e + f;
+    gu8 *qa = record_ptr(uni64(ra[0])), *sa = record_ptr(uni64(ra[1]));
+    if constexpr (PB < 0) {
+        if (qa == nullptr) return false;
+        tile(IntC<PA>{}, qa, sa);
+    } else {
+        const int64_t *rb = ra + 4 * (size_t)E;
+        gu8 *qb = record_ptr(uni64(rb[0])), *sb = record_ptr(uni64(rb[1]));
+        if (qb != nullptr) tile(IntC<PB>{}, qb, sb);
+        else if (qa != nullptr) tile(IntC<PA>{}, qa, sa);
+        else return false;
+    }
+    return true;
+}
+
 // Passes of 32 * NMX tokens. NMX = 2 (S = 3 stages of activations): 64 accumulators per lane and 3
 // workgroups per CU, for few tokens per expert (bound by the weight stream). NMX = 4 (S = 2): the
 // conversion of a weight row, as much VALU work as the MFMAs of 64 tokens take, is shared by 128,
@@ -585,13 +612,13 @@ template <int NMX> struct GgPass {
 // gate rows, subtile 1 = up rows. x: fp16 in operand order with exponents xe (see prep_row). Writes
 // h16 (pairs, I): h = silu(gate) * up as fp16 times 2^-eb in operand order, hbe (pairs, I / 32): eb.
 // ---------------------------------------------------------------------------------------
-template <int PREC, int NMX>
+template <int PA, int PB, int NMX>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GgPass<NMX>::WPE, GgPass<NMX>::WPE))) void k_gemm_up(
     const uint16_t *__restrict__ x, uint32_t xbytes, const int *__restrict__ xe, int H, int I, int k, const int4 *__restrict__ units,
-    const int32_t *__restrict__ sorted_pos, const int64_t *__restrict__ tab, uint16_t *__restrict__ h16,
+    const int32_t *__restrict__ sorted_pos, const int64_t *__restrict__ tab, int E, uint16_t *__restrict__ h16,
     int8_t *__restrict__ hbe, DeqK dk) {
-    constexpr int CK = GgPrec<PREC>::CK, TOK = GgPass<NMX>::TOK, S = GgPass<NMX>::S;
-    __shared__ GgUpShared<S * TOK * CK, TOK> sh;
+    constexpr int TOK = GgPass<NMX>::TOK, S = GgPass<NMX>::S, CKX = gg_ck(PA, PB);
+    __shared__ GgUpShared<S * TOK * CKX, TOK> sh;
     uint16_t *s_a = sh.a;
     int *s_e = sh.e;
     const int NB = I / 128;
@@ -599,70 +626,71 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GgPass<NMX>
     if (!tile_of(blockIdx.x, units[0].x, NB, u, nb)) return;
     const int4 un = units[1 + u];
     const int e = un.x, p0 = un.y, mn = un.z, nm = (mn + 31) / 32;
-    gu8 *qb = record_ptr(uni64(tab[4 * (size_t)e + 0]));
-    gu8 *sb = record_ptr(uni64(tab[4 * (size_t)e + 1]));
-    if (qb == nullptr) return;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, j = lane & 31, h = lane >> 5;
     const int col = nb * 128 + 32 * wave + j;
-    uint32_t qo[2], so[2];
-    gemm_rows<PREC>(col, H, h, qo[0], so[0]);
-    gemm_rows<PREC>(I + col, H, h, qo[1], so[1]);
-    const int nch = H / CK;
     const rsrc_t xbuf = buffer_of(x, xbytes);
     const int colp = (col & ~7) | ((col & 3) << 1) | ((col >> 2) & 1);  // operand order within 8
     const int NB32 = I / 32;
-    const int32_t *sp = sorted_pos + p0;
-    if (tid < TOK) s_e[tid] = tid < mn ? xe[(uint32_t)sp[tid] / (uint32_t)k] : 0;
-    f32x16 d[NMX][2];
+    auto tile = [&](auto pc, gu8 *qb, gu8 *sb) {
+        constexpr int PREC = decltype(pc)::value, CK = GgPrec<PREC>::CK;
+        uint32_t qo[2], so[2];
+        gemm_rows<PREC>(col, H, h, qo[0], so[0]);
+        gemm_rows<PREC>(I + col, H, h, qo[1], so[1]);
+        const int nch = H / CK;
+        const int32_t *sp = sorted_pos + p0;
+        if (tid < TOK) s_e[tid] = tid < mn ? xe[(uint32_t)sp[tid] / (uint32_t)k] : 0;
+        f32x16 d[NMX][2];
 #pragma unroll
-    for (int a = 0; a < NMX; ++a)
+        for (int a = 0; a < NMX; ++a)
 #pragma unroll
-        for (int b = 0; b < 2; ++b) d[a][b] = f32x16{};
-    auto loop = [&](auto nmc) {
-        constexpr int NM = decltype(nmc)::value, NA = AStage<CK>::per_wave(NM);
-        uint32_t ao[NA];
+            for (int b = 0; b < 2; ++b) d[a][b] = f32x16{};
+        auto loop = [&](auto nmc) {
+            constexpr int NM = decltype(nmc)::value, NA = AStage<CK>::per_wave(NM);
+            uint32_t ao[NA];
 #pragma unroll
-        for (int q = 0; q < NA; ++q) {
-            int blk;
-            const int r = astage_row<CK, NM>(q, blk);  // rows past the pass read its first row: never stored
-            ao[q] = (uint32_t)sp[r < mn ? r : 0] / (uint32_t)k * (uint32_t)(H * 2) + 16u * blk;
+            for (int q = 0; q < NA; ++q) {
+                int blk;
+                const int r = astage_row<CK, NM>(q, blk);  // rows past the pass read its first row: never stored
+                ao[q] = (uint32_t)sp[r < mn ? r : 0] / (uint32_t)k * (uint32_t)(H * 2) + 16u * blk;
+            }
+            k_loop<PREC, NMX, S, NM, false, true>(qb, sb, qo, so, nch, xbuf, ao, s_a,
+                                                  nullptr, dk, d);
+        };
+        if (nm == 1) loop(IntC<1>{});
+        else if (nm == 2) loop(IntC<2>{});
+        else if constexpr (NMX == 4) {
+            if (nm == 3) loop(IntC<3>{});
+            else loop(IntC<4>{});
         }
-        k_loop<PREC, NMX, S, NM, false, true>(qb, sb, qo, so, nch, xbuf, ao, s_a,
-                                              nullptr, dk, d);
-    };
-    if (nm == 1) loop(IntC<1>{});
-    else if (nm == 2) loop(IntC<2>{});
-    else if constexpr (NMX == 4) {
-        if (nm == 3) loop(IntC<3>{});
-        else loop(IntC<4>{});
-    }
-    // epilogue: h = silu(gate) * up (scaled back by the token's 2^e); per token the largest
-    // |h| of the wave's 32 columns (one half of the wave) sets the block exponent eb. SiLU from
-    // the hardware's exp2 and reciprocal (about 1 ulp of fp32 each; h is then rounded to fp16)
-    // (branch-free first loop: the 16 lane reductions of a tile interleave)
+        // epilogue: h = silu(gate) * up (scaled back by the token's 2^e); per token the largest
+        // |h| of the wave's 32 columns (one half of the wave) sets the block exponent eb. SiLU from
+        // the hardware's exp2 and reciprocal (about 1 ulp of fp32 each; h is then rounded to fp16)
+        // (branch-free first loop: the 16 lane reductions of a tile interleave)
 #pragma unroll
-    for (int mt = 0; mt < NMX; ++mt) {
-        if (mt >= nm) break;
+        for (int mt = 0; mt < NMX; ++mt) {
+            if (mt >= nm) break;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int tok = mt * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
-            const int ex = s_e[tok];
-            const float hv = silu_mul_fast(__builtin_amdgcn_ldexpf(d[mt][0][r], ex), __builtin_amdgcn_ldexpf(d[mt][1][r], ex));
-            d[mt][0][r] = hv;
-            d[mt][1][r] = half_max(fabsf(hv));
-        }
-        uint16_t *hr = h16 + (size_t)(p0 + mt * 32 + 4 * h) * I + colp;
-        int8_t *er = hbe + (size_t)(p0 + mt * 32 + 4 * h) * NB32 + (col >> 5);
+            for (int r = 0; r < 16; ++r) {
+                const int tok = mt * 32 + 8 * (r >> 2) + 4 * h + (r & 3);
+                const int ex = s_e[tok];
+                const float hv = silu_mul_fast(__builtin_amdgcn_ldexpf(d[mt][0][r], ex), __builtin_amdgcn_ldexpf(d[mt][1][r], ex));
+                d[mt][0][r] = hv;
+                d[mt][1][r] = half_max(fabsf(hv));
+            }
+            uint16_t *hr = h16 + (size_t)(p0 + mt * 32 + 4 * h) * I + colp;
+            int8_t *er = hbe + (size_t)(p0 + mt * 32 + 4 * h) * NB32 + (col >> 5);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int tr = 8 * (r >> 2) + (r & 3);
-            const int eb = row_exp(d[mt][1][r]);
-            if (mt * 32 + 4 * h + tr < mn) {
-                hr[(uint32_t)(tr * I)] = f32_to_f16_rne(__builtin_amdgcn_ldexpf(d[mt][0][r], -eb));
-                if (j == 0) er[(uint32_t)(tr * NB32)] = (int8_t)eb;
+            for (int r = 0; r < 16; ++r) {
+                const int tr = 8 * (r >> 2) + (r & 3);
+                const int eb = row_exp(d[mt][1][r]);
+                if (mt * 32 + 4 * h + tr < mn) {
+                    hr[(uint32_t)(tr * I)] = f32_to_f16_rne(__builtin_amdgcn_ldexpf(d[mt][0][r], -eb));
+                    if (j == 0) er[(uint32_t)(tr * NB32)] = (int8_t)eb;
+                }
             }
         }
-    }
+    };
+    gg_tables<PA, PB>(tab, E, e, 0, tile);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1106,13 +1134,13 @@ __global__ __launch_bounds__(256) void k_gemv_down2(const float *__restrict__ hb
 // int4 rows at 64-token passes: 3 waves per SIMD spill (54 us against 48 with 2 at d_model 2048, d_ff
 // 768, 128 experts, 512 tokens); the other kinds fit (fp8 at 512 experts: 127 us with 3, 134 with 2)
 constexpr int gg_down_wpe(int prec, int nmx) { return nmx == 2 && prec != MOEHIP_PREC_INT4 ? 3 : 2; }
-template <int PREC, int NMX, bool EVEN>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(gg_down_wpe(PREC, NMX), gg_down_wpe(PREC, NMX)))) void k_gemm_down(
+template <int PA, int PB, int NMX, bool EVEN>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(gg_down_wpe(PB < 0 ? PA : PB, NMX), gg_down_wpe(PB < 0 ? PA : PB, NMX)))) void k_gemm_down(
     const uint16_t *__restrict__ h16, const int8_t *__restrict__ hbe, int H, int I, const int4 *__restrict__ units,
-    const int32_t *__restrict__ sorted_pos, const int64_t *__restrict__ tab, const float *__restrict__ w,
+    const int32_t *__restrict__ sorted_pos, const int64_t *__restrict__ tab, int E, const float *__restrict__ w,
     float *__restrict__ y, DeqK dk, int zero_missing) {
-    constexpr int CK = GgPrec<PREC>::CK, TOK = GgPass<NMX>::TOK, S = GgPass<NMX>::S, TPT = 256 / TOK;
-    __shared__ GgDownShared<S * TOK * CK, TOK> sh;
+    constexpr int TOK = GgPass<NMX>::TOK, S = GgPass<NMX>::S, TPT = 256 / TOK, CKX = gg_ck(PA, PB);
+    __shared__ GgDownShared<S * TOK * CKX, TOK> sh;
     uint16_t *s_a = sh.a, *s_x = sh.x;
     float *s_f = sh.f;
     const int NB = H / GG_ROWS;
@@ -1121,86 +1149,85 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(gg_down_wpe
     const int4 un = units[1 + u];
     const int e = un.x, p0 = un.y, mn = un.z, nm = (mn + 31) / 32;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, j = lane & 31, h = lane >> 5;
-    gu8 *qb = record_ptr(uni64(tab[4 * (size_t)e + 2]));
-    gu8 *sb = record_ptr(uni64(tab[4 * (size_t)e + 3]));
     const int row0 = nb * GG_ROWS + 64 * wave + j;
-    if (qb == nullptr) {  // expert not resident (single-table launches): its pairs contribute nothing
-        if (zero_missing)
-            for (int i = tid; i < mn * GG_ROWS; i += 256)
-                y[(size_t)(p0 + i / GG_ROWS) * H + nb * GG_ROWS + i % GG_ROWS] = 0.f;
-        return;
-    }
-    uint32_t qo[2], so[2];
-    gemm_rows<PREC>(row0, I, h, qo[0], so[0]);
-    gemm_rows<PREC>(row0 + 32, I, h, qo[1], so[1]);
-    const int stok = tid / TPT, part = tid % TPT;
-    const bool sok = stok < mn;
-    const size_t pr = (size_t)(p0 + (sok ? stok : 0));
-    // the pair's largest block exponent: the TPT threads of the pair take every TPT-th dword (4
-    // blocks), then the largest over them (DPP)
-    const int ND = I / 128;
-    const uint32_t *eb4 = reinterpret_cast<const uint32_t *>(hbe + pr * (I / 32));
-    int emax = -1000;
-    for (int i0 = part; i0 < ND; i0 += TPT) {
-        const int v = (int)eb4[i0];
-        emax = max(max(emax, max((v << 24) >> 24, (v << 16) >> 24)), max((v << 8) >> 24, v >> 24));
-    }
-    emax = max(emax, dpp_i<0xB1>(emax));
-    if constexpr (TPT == 4) emax = max(emax, dpp_i<0x4E>(emax));
-    if (part == 0) s_f[stok] = sok ? w[sorted_pos[pr]] * ldexpf(1.0f, emax) : 0.f;
-    f32x16 d[NMX][2];
-#pragma unroll
-    for (int a = 0; a < NMX; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) d[a][b] = f32x16{};
-    auto loop = [&](auto nmc) {
-        constexpr int NM = decltype(nmc)::value, NA = AStage<CK>::per_wave(NM);
-        uint32_t ao[NA];
-#pragma unroll
-        for (int q = 0; q < NA; ++q) {
-            int blk;
-            const int r = astage_row<CK, NM>(q, blk);
-            ao[q] = (uint32_t)(r < mn ? r : 0) * (uint32_t)(I * 2) + 16u * blk;
+    auto tile = [&](auto pc, gu8 *qb, gu8 *sb) {
+        constexpr int PREC = decltype(pc)::value, CK = GgPrec<PREC>::CK;
+        uint32_t qo[2], so[2];
+        gemm_rows<PREC>(row0, I, h, qo[0], so[0]);
+        gemm_rows<PREC>(row0 + 32, I, h, qo[1], so[1]);
+        const int stok = tid / TPT, part = tid % TPT;
+        const bool sok = stok < mn;
+        const size_t pr = (size_t)(p0 + (sok ? stok : 0));
+        // the pair's largest block exponent: the TPT threads of the pair take every TPT-th dword (4
+        // blocks), then the largest over them (DPP)
+        const int ND = I / 128;
+        const uint32_t *eb4 = reinterpret_cast<const uint32_t *>(hbe + pr * (I / 32));
+        int emax = -1000;
+        for (int i0 = part; i0 < ND; i0 += TPT) {
+            const int v = (int)eb4[i0];
+            emax = max(max(emax, max((v << 24) >> 24, (v << 16) >> 24)), max((v << 8) >> 24, v >> 24));
         }
-#pragma unroll 1
-        for (int k0 = 0; k0 < I; k0 += GG_SEG) {
-            const int kn = min(GG_SEG, I - k0);
-            if (k0 != 0) __syncthreads();  // the previous segment's factors have been read
-            for (int i0 = part; i0 < kn / 128; i0 += TPT) {
-                const int v = (int)eb4[k0 / 128 + i0];
-                const int eb[4] = {(v << 24) >> 24, (v << 16) >> 24, (v << 8) >> 24, v >> 24};
+        emax = max(emax, dpp_i<0xB1>(emax));
+        if constexpr (TPT == 4) emax = max(emax, dpp_i<0x4E>(emax));
+        if (part == 0) s_f[stok] = sok ? w[sorted_pos[pr]] * ldexpf(1.0f, emax) : 0.f;
+        f32x16 d[NMX][2];
 #pragma unroll
-                for (int q = 0; q < 4; ++q) s_x[(4 * i0 + q) * TOK + stok] = (uint16_t)pow2_h(eb[q] - emax);
+        for (int a = 0; a < NMX; ++a)
+#pragma unroll
+            for (int b = 0; b < 2; ++b) d[a][b] = f32x16{};
+        auto loop = [&](auto nmc) {
+            constexpr int NM = decltype(nmc)::value, NA = AStage<CK>::per_wave(NM);
+            uint32_t ao[NA];
+#pragma unroll
+            for (int q = 0; q < NA; ++q) {
+                int blk;
+                const int r = astage_row<CK, NM>(q, blk);
+                ao[q] = (uint32_t)(r < mn ? r : 0) * (uint32_t)(I * 2) + 16u * blk;
             }
-            // (the K loop starts with a barrier)
-            gu8 *qs = qb + (size_t)k0 * GgPrec<PREC>::BITS / 8;
-            gu8 *ss = sb;
-            if constexpr (PREC == MOEHIP_PREC_INT4 || PREC == MOEHIP_PREC_INT8) ss += k0 / GG_KG * 2;
-            else if constexpr (PREC == MOEHIP_PREC_FP8) ss += k0 / 128 * 4;
-            // (the pass's rows from column k0 on)
-            const rsrc_t hbuf = buffer_of(h16 + (size_t)p0 * I + k0, (uint32_t)(mn * I - k0) * 2u);
-            k_loop<PREC, NMX, S, NM, true, EVEN>(qs, ss, qo, so, kn / CK, hbuf, ao, s_a, s_x, dk, d);
+#pragma unroll 1
+            for (int k0 = 0; k0 < I; k0 += GG_SEG) {
+                const int kn = min(GG_SEG, I - k0);
+                if (k0 != 0) __syncthreads();  // the previous segment's factors have been read
+                for (int i0 = part; i0 < kn / 128; i0 += TPT) {
+                    const int v = (int)eb4[k0 / 128 + i0];
+                    const int eb[4] = {(v << 24) >> 24, (v << 16) >> 24, (v << 8) >> 24, v >> 24};
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) s_x[(4 * i0 + q) * TOK + stok] = (uint16_t)pow2_h(eb[q] - emax);
+                }
+                // (the K loop starts with a barrier)
+                gu8 *qs = qb + (size_t)k0 * GgPrec<PREC>::BITS / 8;
+                gu8 *ss = sb;
+                if constexpr (PREC == MOEHIP_PREC_INT4 || PREC == MOEHIP_PREC_INT8) ss += k0 / GG_KG * 2;
+                else if constexpr (PREC == MOEHIP_PREC_FP8) ss += k0 / 128 * 4;
+                // (the pass's rows from column k0 on)
+                const rsrc_t hbuf = buffer_of(h16 + (size_t)p0 * I + k0, (uint32_t)(mn * I - k0) * 2u);
+                k_loop<PREC, NMX, S, NM, true, EVEN>(qs, ss, qo, so, kn / CK, hbuf, ao, s_a, s_x, dk, d);
+            }
+        };
+        if (nm == 1) loop(IntC<1>{});
+        else if (nm == 2) loop(IntC<2>{});
+        else if constexpr (NMX == 4) {
+            if (nm == 3) loop(IntC<3>{});
+            else loop(IntC<4>{});
+        }
+#pragma unroll
+        for (int mt = 0; mt < NMX; ++mt) {
+            if (mt >= nm) break;
+            float *yr = y + (size_t)(p0 + mt * 32 + 4 * h) * H + row0;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int tr = 8 * (r >> 2) + (r & 3);
+                if (mt * 32 + 4 * h + tr >= mn) continue;
+                const float f = s_f[mt * 32 + 4 * h + tr];
+                yr[(uint32_t)(tr * H)] = f * d[mt][0][r];
+                yr[(uint32_t)(tr * H) + 32] = f * d[mt][1][r];
+            }
         }
     };
-    if (nm == 1) loop(IntC<1>{});
-    else if (nm == 2) loop(IntC<2>{});
-    else if constexpr (NMX == 4) {
-        if (nm == 3) loop(IntC<3>{});
-        else loop(IntC<4>{});
-    }
-#pragma unroll
-    for (int mt = 0; mt < NMX; ++mt) {
-        if (mt >= nm) break;
-        float *yr = y + (size_t)(p0 + mt * 32 + 4 * h) * H + row0;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int tr = 8 * (r >> 2) + (r & 3);
-            if (mt * 32 + 4 * h + tr >= mn) continue;
-            const float f = s_f[mt * 32 + 4 * h + tr];
-            yr[(uint32_t)(tr * H)] = f * d[mt][0][r];
-            yr[(uint32_t)(tr * H) + 32] = f * d[mt][1][r];
-        }
-    }
+    // expert not resident (single-table launches): its pairs contribute nothing
+    if (!gg_tables<PA, PB>(tab, E, e, 2, tile) && zero_missing)
+        for (int i = tid; i < mn * GG_ROWS; i += 256)
+            y[(size_t)(p0 + i / GG_ROWS) * H + nb * GG_ROWS + i % GG_ROWS] = 0.f;
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1998,35 +2025,35 @@ extern "C" size_t moehip_grouped_gemm_workspace_bytes(int T, int k, int H, int I
 // the device; an expert of any size is correct in either).
 static int gg_tokens(int NP, int E) { return NP >= 48 * (int64_t)E ? 128 : 64; }
 
-template <int PREC>
+template <int PA, int PB = -1>
 static void launch_up(int tok, int MU, hipStream_t st, const uint16_t *x, uint32_t xbytes, const int *xe, int H, int I, int k,
-                      const int4 *units, const int32_t *sorted_pos, const int64_t *tab, uint16_t *h16, int8_t *hbe,
+                      const int4 *units, const int32_t *sorted_pos, const int64_t *tab, int E, uint16_t *h16, int8_t *hbe,
                       DeqK dk) {
     const dim3 g((MU + 7) / 8 * 8 * (I / 128));
-    if (tok == 128) hipLaunchKernelGGL((k_gemm_up<PREC, 4>), g, dim3(256), 0, st, x, xbytes, xe, H, I, k, units, sorted_pos, tab, h16, hbe, dk);
-    else hipLaunchKernelGGL((k_gemm_up<PREC, 2>), g, dim3(256), 0, st, x, xbytes, xe, H, I, k, units, sorted_pos, tab, h16, hbe, dk);
+    if (tok == 128) hipLaunchKernelGGL((k_gemm_up<PA, PB, 4>), g, dim3(256), 0, st, x, xbytes, xe, H, I, k, units, sorted_pos, tab, E, h16, hbe, dk);
+    else hipLaunchKernelGGL((k_gemm_up<PA, PB, 2>), g, dim3(256), 0, st, x, xbytes, xe, H, I, k, units, sorted_pos, tab, E, h16, hbe, dk);
 }
-template <int PREC, bool EVEN>
+template <int PA, int PB, bool EVEN>
 static void launch_down_e(int tok, int MU, hipStream_t st, const uint16_t *h16, const int8_t *hbe, int H, int I,
-                          const int4 *units, const int32_t *sorted_pos, const int64_t *tab, const float *w, float *y,
+                          const int4 *units, const int32_t *sorted_pos, const int64_t *tab, int E, const float *w, float *y,
                           DeqK dk, int zero_missing) {
     const dim3 g((MU + 7) / 8 * 8 * (H / GG_ROWS));
     if (tok == 128)
-        hipLaunchKernelGGL((k_gemm_down<PREC, 4, EVEN>), g, dim3(256), 0, st, h16, hbe, H, I, units, sorted_pos, tab, w, y, dk, zero_missing);
+        hipLaunchKernelGGL((k_gemm_down<PA, PB, 4, EVEN>), g, dim3(256), 0, st, h16, hbe, H, I, units, sorted_pos, tab, E, w, y, dk, zero_missing);
     else
-        hipLaunchKernelGGL((k_gemm_down<PREC, 2, EVEN>), g, dim3(256), 0, st, h16, hbe, H, I, units, sorted_pos, tab, w, y, dk, zero_missing);
+        hipLaunchKernelGGL((k_gemm_down<PA, PB, 2, EVEN>), g, dim3(256), 0, st, h16, hbe, H, I, units, sorted_pos, tab, E, w, y, dk, zero_missing);
 }
 template <int PREC>
 static void launch_down(int tok, int MU, hipStream_t st, const uint16_t *h16, const int8_t *hbe, int H, int I,
-                        const int4 *units, const int32_t *sorted_pos, const int64_t *tab, const float *w, float *y,
+                        const int4 *units, const int32_t *sorted_pos, const int64_t *tab, int E, const float *w, float *y,
                         DeqK dk, int zero_missing) {
     if constexpr (PREC == MOEHIP_PREC_INT4) {  // the other kinds have an even number of chunks for any I
         if (I % 256 != 0) {
-            launch_down_e<PREC, false>(tok, MU, st, h16, hbe, H, I, units, sorted_pos, tab, w, y, dk, zero_missing);
+            launch_down_e<PREC, -1, false>(tok, MU, st, h16, hbe, H, I, units, sorted_pos, tab, E, w, y, dk, zero_missing);
             return;
         }
     }
-    launch_down_e<PREC, true>(tok, MU, st, h16, hbe, H, I, units, sorted_pos, tab, w, y, dk, zero_missing);
+    launch_down_e<PREC, -1, true>(tok, MU, st, h16, hbe, H, I, units, sorted_pos, tab, E, w, y, dk, zero_missing);
 }
 
 // the persistent FFN of one record table: plan, then one workgroup per CU slot (at most)
@@ -2320,29 +2347,45 @@ static int gg_run(int P, const int *precs, const int64_t *tabs, const void *x, i
     // the MFMA up tiles write h as fp16 with a power of two per (pair, 32 columns); the GEMVs fp32
     uint16_t *h16 = reinterpret_cast<uint16_t *>(wsb + L.h16);
     int8_t *hbe = reinterpret_cast<int8_t *>(wsb + L.hbe);
-    for (int p = 0; p < P && !gemv && !fused; ++p) {
+    // a 16-bit + int4 store, the pair a precision policy is used with: both tables in one up and one
+    // down launch (faster at every mix measured, 32 to 1024 tokens: see gg_tables). Other pairs, and an
+    // odd number of int4 chunks, keep a launch per table rather than twice the instantiations
+    const bool pair = !gemv && !fused && P == 2 && precs[1] == MOEHIP_PREC_INT4 && I % 256 == 0 &&
+                      (precs[0] == MOEHIP_PREC_F16 || precs[0] == MOEHIP_PREC_BF16);
+    const bool tiles = !gemv && !fused && !pair;
+    if (pair) {
+        const uint32_t xb = (uint32_t)((size_t)T * H * 2);
+        if (precs[0] == MOEHIP_PREC_F16) {
+            launch_up<MOEHIP_PREC_F16, MOEHIP_PREC_INT4>(tok, MU, st, x16, xb, xe, H, I, k, units, sorted_pos, tabs, E, h16, hbe, dk);
+            launch_down_e<MOEHIP_PREC_F16, MOEHIP_PREC_INT4, true>(tok, MU, st, h16, hbe, H, I, units, sorted_pos, tabs, E, w, y, dk, 0);
+        } else {
+            launch_up<MOEHIP_PREC_BF16, MOEHIP_PREC_INT4>(tok, MU, st, x16, xb, xe, H, I, k, units, sorted_pos, tabs, E, h16, hbe, dk);
+            launch_down_e<MOEHIP_PREC_BF16, MOEHIP_PREC_INT4, true>(tok, MU, st, h16, hbe, H, I, units, sorted_pos, tabs, E, w, y, dk, 0);
+        }
+    }
+    for (int p = 0; p < P && tiles; ++p) {
         const int64_t *tab = tabs + (size_t)p * E * 4;
         switch (precs[p]) {
-            case MOEHIP_PREC_INT4: launch_up<MOEHIP_PREC_INT4>(tok, MU, st, x16, (uint32_t)((size_t)T * H * 2), xe, H, I, k, units, sorted_pos, tab, h16, hbe, dk); break;
-            case MOEHIP_PREC_INT8: launch_up<MOEHIP_PREC_INT8>(tok, MU, st, x16, (uint32_t)((size_t)T * H * 2), xe, H, I, k, units, sorted_pos, tab, h16, hbe, dk); break;
-            case MOEHIP_PREC_FP8: launch_up<MOEHIP_PREC_FP8>(tok, MU, st, x16, (uint32_t)((size_t)T * H * 2), xe, H, I, k, units, sorted_pos, tab, h16, hbe, dk); break;
-            case MOEHIP_PREC_F16: launch_up<MOEHIP_PREC_F16>(tok, MU, st, x16, (uint32_t)((size_t)T * H * 2), xe, H, I, k, units, sorted_pos, tab, h16, hbe, dk); break;
-            default: launch_up<MOEHIP_PREC_BF16>(tok, MU, st, x16, (uint32_t)((size_t)T * H * 2), xe, H, I, k, units, sorted_pos, tab, h16, hbe, dk); break;
+            case MOEHIP_PREC_INT4: launch_up<MOEHIP_PREC_INT4>(tok, MU, st, x16, (uint32_t)((size_t)T * H * 2), xe, H, I, k, units, sorted_pos, tab, E, h16, hbe, dk); break;
+            case MOEHIP_PREC_INT8: launch_up<MOEHIP_PREC_INT8>(tok, MU, st, x16, (uint32_t)((size_t)T * H * 2), xe, H, I, k, units, sorted_pos, tab, E, h16, hbe, dk); break;
+            case MOEHIP_PREC_FP8: launch_up<MOEHIP_PREC_FP8>(tok, MU, st, x16, (uint32_t)((size_t)T * H * 2), xe, H, I, k, units, sorted_pos, tab, E, h16, hbe, dk); break;
+            case MOEHIP_PREC_F16: launch_up<MOEHIP_PREC_F16>(tok, MU, st, x16, (uint32_t)((size_t)T * H * 2), xe, H, I, k, units, sorted_pos, tab, E, h16, hbe, dk); break;
+            default: launch_up<MOEHIP_PREC_BF16>(tok, MU, st, x16, (uint32_t)((size_t)T * H * 2), xe, H, I, k, units, sorted_pos, tab, E, h16, hbe, dk); break;
         }
     }
     if (two) launch_gv2(precs, 0, items, NP, st, hb, nullptr, H, I, k, offsets, sorted_pos, tabs, E, y, w, dk);
     for (int p = 0; p < P && gemv && !two; ++p)
         launch_gv_prec(precs[p], 0, items + (size_t)p * (NP + 1), NP, st, hb, nullptr, H, I, k, offsets, sorted_pos, tabs + (size_t)p * E * 4,
                        y, w, dk);
-    for (int p = 0; p < P && !gemv && !fused; ++p) {
+    for (int p = 0; p < P && tiles; ++p) {
         const int64_t *tab = tabs + (size_t)p * E * 4;
         const int zm = zero_missing && P == 1;
         switch (precs[p]) {
-            case MOEHIP_PREC_INT4: launch_down<MOEHIP_PREC_INT4>(tok, MU, st, h16, hbe, H, I, units, sorted_pos, tab, w, y, dk, zm); break;
-            case MOEHIP_PREC_INT8: launch_down<MOEHIP_PREC_INT8>(tok, MU, st, h16, hbe, H, I, units, sorted_pos, tab, w, y, dk, zm); break;
-            case MOEHIP_PREC_FP8: launch_down<MOEHIP_PREC_FP8>(tok, MU, st, h16, hbe, H, I, units, sorted_pos, tab, w, y, dk, zm); break;
-            case MOEHIP_PREC_F16: launch_down<MOEHIP_PREC_F16>(tok, MU, st, h16, hbe, H, I, units, sorted_pos, tab, w, y, dk, zm); break;
-            default: launch_down<MOEHIP_PREC_BF16>(tok, MU, st, h16, hbe, H, I, units, sorted_pos, tab, w, y, dk, zm); break;
+            case MOEHIP_PREC_INT4: launch_down<MOEHIP_PREC_INT4>(tok, MU, st, h16, hbe, H, I, units, sorted_pos, tab, E, w, y, dk, zm); break;
+            case MOEHIP_PREC_INT8: launch_down<MOEHIP_PREC_INT8>(tok, MU, st, h16, hbe, H, I, units, sorted_pos, tab, E, w, y, dk, zm); break;
+            case MOEHIP_PREC_FP8: launch_down<MOEHIP_PREC_FP8>(tok, MU, st, h16, hbe, H, I, units, sorted_pos, tab, E, w, y, dk, zm); break;
+            case MOEHIP_PREC_F16: launch_down<MOEHIP_PREC_F16>(tok, MU, st, h16, hbe, H, I, units, sorted_pos, tab, E, w, y, dk, zm); break;
+            default: launch_down<MOEHIP_PREC_BF16>(tok, MU, st, h16, hbe, H, I, units, sorted_pos, tab, E, w, y, dk, zm); break;
         }
     }
     if (xdtype == MOEHIP_DT_F16)

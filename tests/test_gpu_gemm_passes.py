@@ -41,3 +41,27 @@ def test_passes_and_chunks(dev, prec, dtype, tok, I):
     mats = {e: _mats(st, prec, 0, e) for e in range(E) if counts[e]}
     ref = O.moe_layer_grouped(x.float().numpy(), idx.numpy(), w.numpy().astype(np.float64), lambda e: mats[e])
     assert_layer_close(out.float().cpu().numpy(), ref, dtype)
+
+
+@pytest.mark.parametrize("I", [384, 512])
+@pytest.mark.parametrize("tok", list(COUNTS))
+@pytest.mark.parametrize("hi", ["fp16", "bf16", "int8"])
+def test_two_precisions(dev, hi, tok, I):
+    """Experts of both precisions in one batch: 16-bit + int4 in one launch, the odd number of int4
+    chunks (I = 384) and int8 + int4 in a launch each."""
+    H, counts = 512, COUNTS[tok]
+    E, T = len(counts), sum(counts)
+    st = _store(dev, [hi, "int4"], H, I, E, 37)
+    g = torch.Generator().manual_seed(I + len(counts))
+    idx = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(T, generator=g)].view(T, 1)
+    w = torch.where(idx % 3 == 0, 0.8, 0.2).float()  # every third expert's tokens vote for the first precision
+    x = torch.randn(T, H, generator=g).half()
+    gl = GroupedLayer(st, 1, T, PrecisionPolicy("weight", t1=0.5, upgrade=False), x.dtype, gemv_tokens=0)
+    out = torch.zeros(T, H, dtype=x.dtype, device=dev)
+    gl.layer(0, x.to(dev), out, idx.to(dev), w.to(dev))
+    torch.cuda.synchronize()
+    info = gl.info[0].cpu().tolist()
+    assert [info[e] for e in range(E) if counts[e]] == [0 if e % 3 == 0 else 1 for e in range(E) if counts[e]]
+    mats = {e: _mats(st, hi if e % 3 == 0 else "int4", 0, e) for e in range(E) if counts[e]}
+    ref = O.moe_layer_grouped(x.float().numpy(), idx.numpy(), w.numpy().astype(np.float64), lambda e: mats[e])
+    assert_layer_close(out.float().cpu().numpy(), ref, x.dtype)
