@@ -452,8 +452,8 @@ int moehip_batch_vote(const int32_t *levels, int E, int has_shared, const int32_
                       int32_t *rank, float *info, float *miss, void *stream);
 
 /*
- * moehip_batch_levels + moehip_dispatch + moehip_batch_vote in one launch (one workgroup; the same
- * arguments and results): w32 / idx are (T, ks) with the shared expert (id E) as the last slot
+ * moehip_batch_levels + moehip_dispatch + moehip_batch_vote (the same arguments and results) in one
+ * launch of one workgroup; above 64 tokens the levels are a launch over the whole chip before it: w32 / idx are (T, ks) with the shared expert (id E) as the last slot
  * when has_shared. T * ks <= 65536, E + has_shared <= 1024. For batched decode, where each of
  * those steps is a few microseconds of launch latency. items (P * (T * ks + 1) int32, or NULL):
  * also the work lists of moehip_grouped_gemv_multi, one per record precision (T <= 256).

@@ -1,5 +1,5 @@
-// The dense part in int8 (attention projections, shared experts, the LM head): one-token GEMV and
-// the row-block dequantisation of the multi-token path. Weights (O, K) int8, group scales (O, K/gs)
+// The dense part in int8 (attention projections, shared experts, the LM head): one-token GEMV, the
+// MFMA product of 2 to 256 tokens and the row-block dequantisation for more. Weights (O, K) int8, group scales (O, K/gs)
 // fp16, symmetric (the store's int8 format).
 
 #include "lanevec.hpp"

@@ -52,18 +52,14 @@ typedef gbyte gu8;  // record bytes, global address space (common.hpp)
 __device__ __forceinline__ gu8 *record_ptr(int64_t a) { return gbytes((uint64_t)a); }
 
 constexpr int GG_KG = 64;     // K per scale group
-constexpr int GG_TOK = 64;    // tokens per pass (two 32-token M tiles)
+constexpr int GG_TOK = 64;    // tokens per pass of the persistent FFN (two 32-token M tiles)
 constexpr int GG_ROWS = 256;  // weight rows per workgroup
 
 // chunk geometry: CK values of K per chunk; a lane half covers CK / 2 of them, which is 32 bytes
 // of its weight row for every record precision (int4: CK 128 = two scale groups, one per half;
-// int8 / fp8: 64; fp16 / bf16: 32). Each of the 256 threads stages CK / 4 fp16 activation values
-// of one token (NV 16-byte loads).
+// int8 / fp8: 64; fp16 / bf16: 32)
 template <int CKV> struct GgChunk {
-    static constexpr int CK = CKV;          // K per chunk
-    static constexpr int LDA = CK + 8;      // LDS row stride in halves
-    static constexpr int VPT = CK / 4;      // values staged per thread
-    static constexpr int NV = VPT / 8;      // 16-byte loads per thread
+    static constexpr int LDA = CKV + 8;  // LDS row stride in halves of the persistent FFN's stages
 };
 template <int N> struct IntC { static constexpr int value = N; };
 template <int PREC> struct GgPrec;

@@ -2,7 +2,7 @@
 T > 1 tokens through one layer's experts on the GPU (prefill chunks, batched decode).
 
 Replaces moelab/runtime.py:418-436 (`_run_grouped_tokens`: per expert, expert_ffn on the
-expert's tokens) and runtime.py:352-353 (`out.index_add_(0, tok, y * w)`) for int4 gs64 records:
+expert's tokens) and runtime.py:352-353 (`out.index_add_(0, tok, y * w)`):
 moehip_dispatch sorts the (token, slot) pairs by expert (stable, as runtime.py:459-492), then
 moehip_grouped_gemm runs the gate/up and down GEMMs of every routed expert on MFMA and sums each
 token's slots in slot order. Everything is on the device and capturable; nothing is copied to
@@ -154,7 +154,8 @@ class GroupedLayer:
       3. levels and skip per (token, slot)            (moehip_batch_levels)
       4. expert-sorted dispatch of the kept pairs     (moehip_dispatch)
       5. vote, resident copy, per-precision tables    (moehip_batch_vote)
-         with fused_decide (the default): 3-5 in one launch (moehip_batch_decide), and, when the
+         with fused_decide (the default): 3-5 in one launch (moehip_batch_decide; the levels in a
+         launch of their own above 64 tokens), and, when the
          router runs here on up to route_fused_tokens 16-bit tokens, the top-k, 2, 3-5 and the
          GEMVs' work list in one launch after the logits (moehip_router_logits +
          moehip_batch_route_decide)
