@@ -128,7 +128,8 @@ class GroupedTokens:
 #   fp8   64 experts: 12: 110 / 108, 16: 130 / 113;  128: 16: 116 / 135, 32: 188 / 151;  512: 48: 246 / 247,
 #         64: 308 / 267;  16 top-4 (512): 16: 52 / 59, 32: 76 / 61
 #   fp16  64 experts: 20: 191 / 195, 24: 211 / 197;  16 top-4 (1024): 16: 87 / 101, 32: 121 / 99
-#   fp16 + int4 (weight rule)  64 experts: 16: 129 / 150, 24: 175 / 110;  128: 32: 218 / 284, 48: 291 / 261
+#   fp16 + int4 (weight rule)  64 experts: 14: 102 / 111, 16: 129 / 109, 24: 175 / 90;  128: 28: 164 / 218,
+#         32: 217 / 221, 48: 290 / 200; with more experts at fp16 the line lies further out (all: as fp16)
 GEMV_RATIO_EXTRA = {"int4": (2.0, 93e6), "int8": (2.0, 150e6), "fp8": (1.7, 150e6), "fp16": (2.3, 400e6),
                     "bf16": (2.3, 400e6)}
 
