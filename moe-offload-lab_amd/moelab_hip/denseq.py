@@ -1,6 +1,7 @@
 """The dense part in int8 (moelab/denseq.py): attention projections, shared experts and the LM
 head as int8 weights in groups of 64 with fp16 scales, read directly by a gfx950 GEMV for one
-token, dequantised one block of rows at a time into a scratch matrix for several.
+token and by an MFMA kernel for a few, dequantised one block of rows at a time into a scratch
+matrix for many.
 
 Same names and meaning as moelab's module: `gemv_int8(q, s, x, group_size)`, `QLinear` (a
 drop-in for nn.Linear: `QLinear(q, s, group_size, bias, out_dtype)` and
@@ -13,6 +14,7 @@ from __future__ import annotations
 
 import torch
 import torch.nn as nn
+from torch.autograd.forward_ad import unpack_dual
 
 from . import _lib
 from .store import pick_group_size
@@ -111,17 +113,20 @@ class QLinear(nn.Module):
         return y
 
     def _few(self, x2: torch.Tensor) -> bool:
-        """Whether moehip_dense_gemm_int8 takes these tokens (an input that wants a gradient goes the
-        other way and is refused there, by the out= products)."""
-        return (x2.shape[0] <= FEW_TOKENS and x2.dtype in (torch.float16, torch.bfloat16) and self.group_size == 64
+        """Whether moehip_dense_gemm_int8 takes these tokens (an input or bias that wants a gradient or
+        carries a tangent goes the other way and is refused there, by the out= products)."""
+        if torch.is_grad_enabled() and (x2.requires_grad or (self.bias is not None and self.bias.requires_grad)):
+            return False
+        if unpack_dual(x2).tangent is not None:  # None outside of a dual level
+            return False
+        return (0 < x2.shape[0] <= FEW_TOKENS and x2.device == self.q.device and x2.dtype in (torch.float16, torch.bfloat16) and self.group_size == 64
                 and self.in_features < 1 << 25 and x2.data_ptr() % 16 == 0 and self.q.data_ptr() % 16 == 0
-                and self.q.is_contiguous() and self.s.is_contiguous()
-                and not (x2.requires_grad and torch.is_grad_enabled()))
+                and self.q.is_contiguous() and self.s.is_contiguous())
 
     def _few_tokens(self, x2: torch.Tensor) -> torch.Tensor:
         n = x2.shape[0]
         y = torch.empty(n, self.out_features, dtype=x2.dtype, device=x2.device)
-        bias = None if self.bias is None else self.bias.to(x2.dtype)
+        bias = None if self.bias is None else self.bias.to(x2.dtype).contiguous()
         _lib.call("moehip_dense_gemm_int8", self.q.data_ptr(), self.s.data_ptr(), x2.data_ptr(), _lib.ptr(bias),
                   y.data_ptr(), n, self.out_features, self.in_features, 64, _lib.dt_code(x2.dtype),
                   _lib.stream_of(x2.device))

@@ -169,7 +169,7 @@ def encode_record_(layout: dict, blob: torch.Tensor, gate_up: torch.Tensor, down
 def _padding(layout: dict) -> list[tuple[int, int]]:
     """Byte ranges of a record that no field covers."""
     gaps, end = [], 0
-    for _, shape, dtype, off in layout["fields"]:
+    for _, shape, dtype, off in sorted(layout["fields"], key=lambda f: f[3]):
         if off > end:
             gaps.append((end, off))
         end = off + ELEM_SIZE[dtype] * math.prod(shape)

@@ -67,3 +67,23 @@ def test_dense_gemm_int8_routes(dev):
     assert ql._few(x.half())
     with pytest.raises(RuntimeError):
         ql(x.half().requires_grad_())
+
+
+def test_dense_gemm_int8_other_calls(dev):
+    """No tokens, a strided bias, a trainable bias and a forward-mode tangent: as the dequantised way
+    takes or refuses them."""
+    g = torch.Generator().manual_seed(2)
+    q = torch.randint(-127, 128, (96, 128), generator=g, dtype=torch.int8).to(dev)
+    s = torch.full((96, 2), 1e-3, dtype=torch.float16, device=dev)
+    x = torch.randn(4, 128, generator=g).half().to(dev)
+    bias = torch.randn(192, generator=g).half().to(dev)[::2]
+    ql = D.QLinear(q, s, 64, bias, torch.float16)
+    assert ql(x[:0]).shape == (0, 96) and ql(x.new_zeros(2, 0, 128)).shape == (2, 0, 96)
+    ref = x.double() @ (q.double() * s[0, 0].double()).t() + bias.double()
+    assert ql._few(x) and np.allclose(ql(x).double().cpu(), ref.cpu(), rtol=2e-3, atol=2e-3)
+    with torch.autograd.forward_ad.dual_level():
+        assert not ql._few(torch.autograd.forward_ad.make_dual(x, torch.ones_like(x)))
+    ql.bias.requires_grad_(True)
+    assert not ql._few(x)
+    with pytest.raises(RuntimeError):
+        ql(x)
